@@ -89,6 +89,46 @@ def test_gacc_matches_the_oracle(gpu, quads, slots, blocks, high_bits):
         assert np.array_equal(got2[4 * q: 4 * q + 4], want2), q
 
 
+# 5 quads run one channel per lane, 300 of 4 blocks two and of 8 blocks four;
+# 17 slots leave a ragged last group of 16 entries, 33 a third chunk of 64.
+@pytest.mark.parametrize("quads,slots,blocks", [(5, 17, 1), (5, 33, 8), (300, 17, 4),
+                                                (300, 5, 8), (300, 17, 7)])
+def test_gacc_special_values(gpu, quads, slots, blocks):
+    """Every exponent in w, bw, the scale bytes and the starting accumulators
+    (zeros of both signs, subnormals, 255), a token with no entries at all:
+    overflows, flushes and the guarded arithmetic, bitwise."""
+    rng = np.random.default_rng(slots * 10 + blocks)
+    ddr, list_base, list_bytes, w_stride = build_image(rng, quads, slots, blocks, 40)
+    row = hb.row_token_bytes(blocks)
+    some = rng.random(40) < 0.5  # half of the rows with scale bytes of any value
+    for i in np.nonzero(some)[0]:
+        ddr[i * row + 32 * blocks: i * row + 33 * blocks] = rng.integers(0, 256, blocks)
+    w = ddr[40 * row: list_base].view(np.uint32)
+    odd = rng.random(w.size) < 0.02
+    w[odd] = rng.integers(0, 1 << 32, int(odd.sum()), dtype=np.uint64).astype(np.uint32)
+    lists = ddr[list_base:].reshape(quads, list_bytes)[:, 16:]
+    bw = np.ascontiguousarray(lists).view(np.uint32).reshape(quads, -1)
+    odd = rng.random((quads, bw.shape[1] // 2)) < 0.02
+    bw[:, 1::2][odd] = rng.integers(0, 1 << 32, int(odd.sum()), dtype=np.uint64)
+    bw.reshape(quads, slots, 4, 8)[1, :, 2, 0::2] = 0xFFFFFFFF  # quad 1's token 2: no entries
+    ddr[list_base:].reshape(quads, list_bytes)[:, 16:] = bw.view(np.uint8).reshape(quads, -1)
+    start = random_floats(rng, quads * 4 * 32 * blocks, 120)
+    odd = rng.random(start.size) < 0.1
+    start[odd] = rng.integers(0, 1 << 32, int(odd.sum()), dtype=np.uint64).astype(np.uint32)
+    start[rng.random(start.size) < 0.05] = 0x80000000
+    start[rng.random(start.size) < 0.02] = 0x7F800000
+    start = start.reshape(quads * 4, -1)
+    say("gacc special", dict(quads=quads, slots=slots, blocks=blocks))
+    base, out = dev(ddr), dev(start.view(np.int32)).view(torch.float32)
+    hb.gacc(base, base[list_base:], quads, slots, blocks, w_stride, out, list_stride=list_bytes,
+            accumulate=True, ctx=gpu)
+    got = out.cpu().numpy().view(np.uint32)
+    for q in range(quads):
+        want = oracle.gacc(ddr, list_base + q * list_bytes, slots, blocks, w_stride,
+                           start[4 * q: 4 * q + 4])
+        assert np.array_equal(got[4 * q: 4 * q + 4], want), q
+
+
 @pytest.mark.parametrize("slots,blocks,text", [(1, 9, "GACC with 9 blocks per token"),
                                                (2048, 2, "GACC with 2048 slots"),
                                                (0, 3, "a DMA transfer with 0 rows of 3 words")])
