@@ -215,6 +215,90 @@ __device__ __forceinline__ void EpApplyFast16(uint32_t kind, uint32_t imm, f32x1
   EpApplyFastN<kSerial>(kind, imm, y, x2, p, t);
 }
 
+// EpApply over 4 values of a lane.  The FP32 unit gives the lane formulas'
+// bits except where an operand or a result has exponent field 255 or a
+// product of nonzero operands comes out with field 0 or 1 (it may have
+// rounded up to, or been flushed below, 2^-126), so the hardware form runs
+// first (EpApplyFastN's arithmetic) and a lane that saw such a field takes
+// the integer routines for its 4 values.  About 12 instructions a value and
+// op against 40 with every operation guarded.
+__device__ __forceinline__ bool ProductOdd(uint32_t a, uint32_t b, uint32_t r) {
+  return ExpField(a) != 0 && ExpField(b) != 0 && ExpField(r) <= 1u;
+}
+__device__ __forceinline__ bool TopField(uint32_t x) { return ExpField(x) == 255u; }
+
+// x T(|x|) as ActGateFast, *odd raised where a step may differ from ActGate.
+__device__ __forceinline__ float ActGateChecked(float x, const uint64_t* t, bool* odd) {
+  const float pre = x + 0.0f;
+  const uint32_t bits = __float_as_uint(pre), e = ExpField(bits);
+  const uint32_t sig = Significand(bits);
+  const uint32_t sh = e >= 105u && e <= 129u ? 129u - e : 31u;
+  const uint32_t fixed = e == 130u ? sig << 1 : e < 105u || e > 130u ? 0u : sig >> sh;
+  const uint64_t entry = t[fixed >> 16];
+  const uint32_t ev = (uint32_t)entry, es = (uint32_t)(entry >> 32);
+  const float frac = (float)(fixed & 0xFFFFu) * (1.0f / 65536.0f);
+  const float step = __uint_as_float(es) * frac;
+  float v = __uint_as_float(ev) + step;
+  *odd |= TopField(ev) || TopField(es) || TopField(__float_as_uint(v)) ||
+          ProductOdd(es, __float_as_uint(frac), __float_as_uint(step));
+  v = e >= 131u ? 1.0f : v;
+  const float prod = pre * v;
+  const float y = (__float_as_uint(x) >> 31) ? (-prod + x) + 0.0f : prod + 0.0f;
+  *odd |= TopField(bits) || TopField(__float_as_uint(prod)) || TopField(__float_as_uint(y)) ||
+          ProductOdd(bits, __float_as_uint(v), __float_as_uint(prod));
+  return y;
+}
+
+__device__ __forceinline__ void EpApply4(uint32_t kind, uint32_t imm, f32x4_t& y,
+                                         const f32x4_t& x2, const f32x4_t& p, const uint64_t* t) {
+  f32x4_t r;
+  bool odd = false;
+  switch (kind) {
+    case kEpAct:
+#pragma unroll
+      for (int k = 0; k < 4; ++k) r[k] = ActGateChecked(y[k], t, &odd);
+      break;
+    case kEpActMul:
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float gate = ActGateChecked(y[k], t, &odd);
+        const float prod = gate * x2[k];
+        odd |= TopField(__float_as_uint(x2[k])) || TopField(__float_as_uint(prod)) ||
+               ProductOdd(__float_as_uint(gate), __float_as_uint(x2[k]), __float_as_uint(prod));
+        r[k] = prod + 0.0f;
+      }
+      break;
+    case kEpMulP:
+    case kEpScale:
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float f = kind == kEpScale ? __uint_as_float(imm) : p[k], prod = y[k] * f;
+        odd |= TopField(__float_as_uint(y[k])) || TopField(__float_as_uint(f)) ||
+               TopField(__float_as_uint(prod)) ||
+               ProductOdd(__float_as_uint(y[k]), __float_as_uint(f), __float_as_uint(prod));
+        r[k] = prod + 0.0f;
+      }
+      break;
+    default:  // sums, copies, ReLU
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float b = kind == kEpAdd ? x2[k] : kind == kEpAddP ? p[k] : 0.0f;
+        const float sum = (y[k] + b) + 0.0f;
+        odd |= TopField(__float_as_uint(y[k])) || TopField(__float_as_uint(b)) ||
+               TopField(__float_as_uint(sum));
+        r[k] = kind == kEpRelu ? (sum > 0.0f ? sum : 0.0f) : sum;
+      }
+      break;
+  }
+  if (odd) {
+#pragma unroll 1
+    for (int k = 0; k < 4; ++k)
+      r[k] = __uint_as_float(EpApply(kind, imm, __float_as_uint(y[k]), __float_as_uint(x2[k]),
+                                     __float_as_uint(p[k]), t));
+  }
+  y = r;
+}
+
 // Reads one dword of every 64-byte line of a kernel argument at once, with
 // one wait for all, so the argument reads that follow (scattered over the
 // structure, many behind branches) hit the scalar cache instead of each

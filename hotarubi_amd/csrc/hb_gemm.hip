@@ -6,78 +6,121 @@
 // integer dot product, folded into an FP32 accumulator in block order.
 //
 // Matrix-core mapping.  Per K block the tile's operands are staged in LDS as
-// bf16: A' = q * 2^(ea-127) (its E8M0 scale folded in) and W' = v, the
+// f16: A' = q * 2^d with d = ea - 130 held to [-14, 5], and W' = v, the
 // unscaled weight value.  q (int8) and v (4-bit value) have at most 8
-// significant bits, so A' and W' are exact bf16 values whenever the scale
-// keeps A' normal.  One v_mfma_f32_16x16x32_bf16 with a zero accumulator then
-// covers exactly one K block, and every product and every partial sum it
-// forms is an integer multiple of 2^(ea-127) below 2^17 of that unit:
-// all exactly representable, so the MFMA returns the exact block value up to
-// W's scale.  The ordered fold is one fma per output and block,
-// acc = fma(value, 2^(ew-127+SBIAS), acc): a single rounding of an exact sum
-// (FTZ mode), which is the NPU's RNE add for normal operands; a -0 result
-// can only appear where the NPU has +0 and is fixed once after the fold.
+// significant bits, so A' and W' are exact, normal f16 values.  One
+// v_mfma_f32_16x16x32_f16 with a zero accumulator then covers exactly one K
+// block, and every product and every partial sum it forms is an integer
+// multiple of 2^d below 2^17 of that unit: all exactly representable, so the
+// MFMA returns the exact block value up to the scales.  The ordered fold is
+// one fma per output and block, acc = fma(value, 2^(ew+ea-d-254+SBIAS), acc)
+// with ea - d = 130: a single rounding of an exact sum (FTZ mode), which is
+// the NPU's RNE add for normal operands; a -0 result can only appear where
+// the NPU has +0 and is fixed once after the fold.  Where a row's ea lies
+// outside [116, 135] the rest of its exponent, 2^(ea-130-d), multiplies the
+// block value first (exact): such steps are flagged and take a second copy
+// of the fold.
 //
 // The argument needs every scale byte of the tile in [70, 179] (exponents
 // -57..52) and |initial C| < 2^126: then operands and products stay normal
 // and the fold cannot overflow (steps <= 8192).  A tile that sees anything
 // else recomputes itself with the integer routines of hb_fp32.h, so the
 // result is bit-exact for every input.
-//
-// HB_LINEAR_FAST lets the MFMA accumulate (C = acc) instead of folding each
-// block separately; that changes only the order of the FP32 additions.
+#include <type_traits>
+
 #include "hb_device.h"
 #include "hb_internal.h"
 
 namespace hb {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kThreads = 256;  // 4 waves
-constexpr int kLdsRow = 40;    // bf16 per LDS row: 32 + 8 pad (80 B: conflict-free b128 reads)
-#ifndef HB_CHUNK
-#define HB_CHUNK 2
-#endif
-constexpr int kChunk = HB_CHUNK;  // K blocks per register prefetch chunk
+constexpr int kThreads = 512;  // 8 waves: 4 stage A, 4 stage W, all fold
+constexpr uint32_t kCheck = 8;  // stages between two looks at the rows' scales (even)
 constexpr uint32_t kSafeLo = 70, kSafeHi = 179;
+// What a kernel knows of the planes' modes: all FP4; W8 hi then lo; anything.
+enum : int { kFmtFp4, kFmtW8, kFmtAny };
+constexpr int32_t kAUnit = 130, kAMin = -14, kAMax = 5;  // d = ea - kAUnit, held to [kAMin, kAMax]
 
-// Tile geometry.  kBM x kBN outputs per workgroup; the 4 waves tile it as
-// kWaveM x kWaveN with a kTM x kTN wave tile of 16x16 MFMA tiles.
-template <int kBM, int kBN>
+// Tile geometry.  kBM x kBN outputs per workgroup; the 8 waves tile it as
+// kWaveM x kWaveN with a kTM x kTN wave tile of 16x16 MFMA tiles.  kC: K
+// blocks staged per barrier.  A staging thread has one unit per stage: half a
+// row-block of A (16 of its 32 bytes), or a column-block of W (16 bytes).
+template <int kBM_, int kBN_, int kWaveM, int kC_, int kWavesPerSimd_>
 struct Tile {
-  static constexpr int kTM = kBM >= 64 ? 64 : kBM;
-  static constexpr int kWaveM = kBM / kTM;
-  static constexpr int kWaveN = 4 / kWaveM;
-  static constexpr int kTN = kBN / kWaveN;
+  static constexpr int kWavesPerSimd = kWavesPerSimd_;
+  static constexpr int kBM = kBM_, kBN = kBN_, kC = kC_;
+  static constexpr int kWaveN = 8 / kWaveM;
+  static constexpr int kTM = kBM / kWaveM, kTN = kBN / kWaveN;
   static constexpr int kTI = kTM / 16, kTJ = kTN / 16;
-  static constexpr int kABytes = kBM * 32 / kThreads;  // A bytes a thread stages per block
-  static constexpr int kWBytes = kBN * 16 / kThreads;  // W bytes a thread stages per block
-  static constexpr int kA4 = kABytes / 4, kW4 = kWBytes / 4;
-  static constexpr int kARowThreads = 32 / kABytes, kWColThreads = 16 / kWBytes;
-  static_assert(kWaveM * kWaveN == 4 && kTN == 64, "wave tile is kTM x 64");
-  static_assert(kABytes % 4 == 0 && kWBytes % 4 == 0, "whole dwords per thread");
+  static constexpr int kAUnits = kBM * 2 * kC, kWUnits = kBN * kC;
+  static constexpr int kOutRow = kBN + 4;  // floats per row of the staged outputs
+  static_assert(kTM % 16 == 0 && kTN % 16 == 0, "whole MFMA tiles");
+  static_assert(kAUnits <= 256 && kWUnits <= 256, "a unit per staging thread");
 };
 
-struct Step {
-  uint32_t p, l, b;  // piece, plane, block within the piece
+// LDS: two stages of kC blocks.  A block's operands lie as the MFMAs read
+// them: 16 rows (columns) of one tile are 64 slots of 16 bytes (8 f16), slot
+// Slot(kq, row) for K elements 8 kq .. + 7, so a wave's read covers 64
+// consecutive slots, each once.  Rows of kq 2, 3 are swapped by eights: a
+// staging lane pair writes kq 0 and 2 (or 1 and 3) of a row at once, and the
+// 16 lanes of a write then use 16 different bank groups.
+template <class T>
+struct Lds {
+  static constexpr int kBM = T::kBM, kBN = T::kBN, kC = T::kC;
+  union {
+    struct {
+      uint4 a[2][kC][kBM / 16][64];
+      uint4 w[2][kC][kBN / 16][64];
+    };
+    struct {  // after the K loop
+      float out[kBM * T::kOutRow];
+      uint64_t act[512];  // activation half of TBUF
+    };
+  };
+  float fw[2][kC][kBN];  // 2^(ew + SBIAS + kAUnit - 254) per column and block
+  float fr[2][kC][kBM];  // 2^(ea - kAUnit - d) per row and block
+  uint32_t unsafe, wide;
 };
+__device__ __forceinline__ uint32_t Slot(uint32_t kq, uint32_t row16) {
+  return kq * 16 + (row16 ^ ((kq & 2) * 4));
+}
 
-// The step after s in fold order (pieces, planes, blocks), by selects only:
-// the step loop stays one basic block.
-__device__ __forceinline__ Step Next(const Step& s, const GemmArgs& g) {
-  Step n;
-  const bool wrap_b = s.b + 1 == g.piece_kb[s.p];
-  const bool wrap_l = wrap_b && s.l + 1 == g.n_planes;
-  n.b = wrap_b ? 0u : s.b + 1;
-  n.l = wrap_l ? 0u : (wrap_b ? s.l + 1 : s.l);
-  n.p = wrap_l ? s.p + 1 : s.p;
-  return n;
+// A stage of the fold: up to kC consecutive blocks of one piece and plane,
+// `live` of them; a stage past the end has none.  Its dead blocks repeat the
+// last live one with A staged as zeros, adding +0.
+struct Stage {
+  uint32_t l, blk, live;
+};
+// The stages in fold order (pieces outer, planes inner).
+template <bool kMulti, int kC>
+struct Cursor {
+  uint32_t p = 0, l = 0, b = 0;
+  __device__ __forceinline__ Stage Take(const GemmArgs& g) {
+    const uint32_t kb = g.piece_kb[kMulti ? p : 0], left = b < kb ? kb - b : 0u;
+    const Stage s{l, g.piece_off[kMulti ? p : 0] + min(b, kb - 1), min(left, (uint32_t)kC)};
+    b += kC;
+    if (b >= kb) {  // the next plane or piece; past the last, b stays at kb or more
+      if (l + 1 < g.n_planes) {
+        ++l;
+        b = 0;
+      } else if (kMulti && p + 1 < g.n_pieces) {
+        ++p;
+        l = b = 0;
+      }
+    }
+    return s;
+  }
+};
+template <int kC>
+__device__ __forceinline__ uint32_t StageCount(const GemmArgs& g) {
+  uint32_t n = 0;
+  for (uint32_t p = 0; p < g.n_pieces; ++p) n += (g.piece_kb[p] + kC - 1) / kC;
+  return n * g.n_planes;
 }
 
 template <bool kLinear>
@@ -103,191 +146,170 @@ __device__ __forceinline__ uint32_t* CElem(const GemmArgs& g, uint32_t* c, uint3
   return c + (size_t)word * 32 + (row & 3) * 8 + (col & 7);
 }
 
-// Which bytes of a K block a thread stages.  A: row r (token t of quad
-// q0 + r/4), bytes [aofs, aofs + kABytes) of its 32; W: column col (lane cl
-// of group g0 + col/8), bytes [wofs, wofs + kWBytes) of its 16.  In the
-// 128-row tile, 8 consecutive lanes take 8 consecutive rows at the same
-// byte offset, so their 16-byte LDS stores hit 8 distinct bank groups
-// (80-byte rows: 80 r mod 128 is a permutation of the 16-byte slots).
-template <class T>
-struct Lane {
-  uint32_t r, aofs, col, wofs;
-  __device__ __forceinline__ Lane() {
-    const uint32_t tid = threadIdx.x;
-    if (T::kARowThreads == 2) {
-      r = (tid & 7) + 8 * (tid >> 4);
-      aofs = ((tid >> 3) & 1) * T::kABytes;
-    } else {
-      r = tid / T::kARowThreads;
-      aofs = (tid % T::kARowThreads) * T::kABytes;
-    }
-    if (T::kWColThreads == 2) {
-      col = (tid & 7) + 8 * (tid >> 4);
-      wofs = ((tid >> 3) & 1) * T::kWBytes;
-    } else {
-      col = tid / T::kWColThreads;
-      wofs = (tid % T::kWColThreads) * T::kWBytes;
-    }
-  }
-};
-
-// Raw operand bytes of one K block, as one thread stages them.  Loads are
-// issued unconditionally: rows and columns past the edge of the layer read
-// the last valid quad or group instead, which only feeds outputs that are
-// never stored (rows of a GEMM depend on their own A row, columns on their
-// own W column).  The load count per chunk is static, so the compiler waits
-// on exactly the chunk being consumed while the next one is in flight.
-template <int kA4, int kW4>
+// Raw operand bytes of one stage, as one thread stages them, and the aligned
+// dword that holds their scale byte.  Loads are issued unconditionally: rows
+// and columns past the edge of the layer (and units past the stage's) read
+// the last valid one instead, which only feeds outputs that are never stored
+// (rows of a GEMM depend on their own A row, columns on their own W column).
 struct Staged {
-  uint32_t a[kA4];
-  uint32_t w[kW4];
-  uint32_t sa, sw, plane;
-  bool zero_a;  // a surplus step past the end: A stages as zeros
+  u32x4 v;
+  uint32_t scale;
 };
 
-// Per-thread byte offsets of the staged bytes within a block's words
-// (linear level: A word (q, blk) at (q * a_row + blk) * 144 and W word
-// (grp, blk) at (grp * kb_total + blk) * 144, so the block index only moves
-// a uniform base).
-struct Offsets {
-  uint32_t a, a_scale, w, w_scale;
-};
-
+// Where a thread's staging unit lies: unit u of A is half u % 2 of row u / 2
+// % kBM of the stage's block u / (2 kBM); unit u of W is column u % kBN of
+// block u / kBN.  (8 consecutive lanes read the 128 bytes of a quad's, or a
+// column group's, block.)  Block blk of the unit's operand lies at
+// (blk >> half) * chunk + (blk & half) * codes from the layer's base, its
+// scale dwords at scales in place of codes (DDR words, or panels of two
+// blocks a chunk: WBlockCodes, WBlockScale without a branch).
 template <bool kLinear, class T>
-__device__ __forceinline__ Offsets ThreadOffsets(const GemmArgs& g, const Lane<T>& ln,
-                                                 uint32_t q0, uint32_t g0) {
-  const uint32_t quad = min(q0 + (ln.r >> 2), g.quads - 1), t = ln.r & 3;
-  const uint32_t grp = min(g0 + (ln.col >> 3), g.groups - 1), cl = ln.col & 7;
-  Offsets o;
-  const uint32_t astride = kLinear ? g.a_row * kDdrWord : 0u;
-  const uint32_t wstride = kLinear ? g.kb_total * kDdrWord : 0u;
-  o.a = quad * astride + t * 32 + ln.aofs;
-  o.a_scale = quad * astride + 128 + t;
-  if (kLinear) {  // DDR words or panels (g.w_panels)
-    const WLaneOff wo = WLane(g, grp * 8 + cl);
-    o.w = wo.codes + ln.wofs;
-    o.w_scale = wo.scale + wo.shift / 8;
-  }
-  (void)wstride;
-  if (!kLinear) {  // keep the quad / group for the wrapping on-chip addresses
-    o.a = (quad << 16) | (t * 32 + ln.aofs);
-    o.a_scale = (quad << 16) | (128 + t);
-    o.w = (grp << 16) | (cl * 16 + ln.wofs);
-    o.w_scale = (grp << 16) | (128 + cl);
-  }
-  return o;
-}
-
-template <int kN>
-__device__ __forceinline__ void LoadDwords(const uint8_t* p, uint32_t* out) {
-  if (kN == 4) {
-    const u32x4 v = *reinterpret_cast<const u32x4*>(p);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) out[i] = v[i];
-  } else if (kN == 2) {
-    const u32x2 v = *reinterpret_cast<const u32x2*>(p);
-    out[0] = v[0];
-    out[1] = v[1];
-  } else {
-#pragma unroll
-    for (int i = 0; i < kN; ++i) out[i] = reinterpret_cast<const uint32_t*>(p)[i];
-  }
-}
-
-template <bool kLinear, class T, class S>
-__device__ __forceinline__ void LoadBlock(const GemmArgs& g, const uint8_t* a, const uint8_t* w0,
-                                          const uint8_t* w1, const Offsets& o, const Step& s,
-                                          S& st) {
-  const uint32_t blk = g.piece_off[s.p] + s.b;
-  st.plane = s.l;
-  const uint8_t* w = s.l ? w1 : w0;
-  if (kLinear) {
-    const uint8_t* ab = a + (size_t)blk * kDdrWord;  // uniform
-    LoadDwords<T::kA4>(ab + o.a, st.a);
-    st.sa = ab[o.a_scale];
-    LoadDwords<T::kW4>(w + WBlockCodes(g, blk) + o.w, st.w);  // uniform base + lane offset
-    st.sw = w[WBlockScale(g, blk) + o.w_scale];
-  } else {
-    const uint8_t* aw = AWord<false>(g, a, o.a >> 16, blk);
-    const uint8_t* ww = WWord<false>(g, w, o.w >> 16, blk);
-    if (T::kA4 == 4) {  // ISS ABUF words are 132 B: only 4-byte aligned
-#pragma unroll
-      for (int i = 0; i < 4; ++i) st.a[i] = reinterpret_cast<const uint32_t*>(aw + (o.a & 0xFFFFu))[i];
+struct Lane {
+  bool w;           // stages W (wave-uniform)
+  uint32_t u;       // the unit
+  uint32_t block;   // its block of the stage
+  uint32_t codes, scale, shift;  // its byte offsets in a block's words (linear); scale bit
+  uint32_t line;    // its quad or column group (instruction level)
+  uint32_t half, chunk, c_step, s_step;
+  __device__ __forceinline__ Lane(const GemmArgs& g, uint32_t q0, uint32_t g0) {
+    w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) != 0;
+    u = min(threadIdx.x & 255u, (w ? T::kWUnits : T::kAUnits) - 1u);
+    half = kLinear && w && g.w_panels ? 1u : 0u;
+    chunk = half ? kPanelChunk : kDdrWord;
+    c_step = kPanelCols * 16;
+    s_step = kPanelCols;
+    if (w) {
+      const uint32_t col = u % T::kBN, grp = min(g0 + (col >> 3), g.groups - 1), cl = col & 7;
+      block = u / T::kBN;
+      line = grp;
+      if (kLinear) {
+        const WLaneOff wo = WLane(g, grp * 8 + cl);
+        codes = wo.codes;
+        scale = wo.scale;
+        shift = wo.shift;
+      } else {
+        codes = cl * 16;
+        scale = 128 + (cl & 4);
+        shift = 8 * (cl & 3);
+      }
     } else {
-      LoadDwords<T::kA4>(aw + (o.a & 0xFFFFu), st.a);
+      const uint32_t r = u / 2 % T::kBM, quad = min(q0 + (r >> 2), g.quads - 1);
+      block = u / (2 * T::kBM);
+      line = quad;
+      codes = (kLinear ? quad * g.a_row * kDdrWord : 0u) + (r & 3) * 32 + (u % 2) * 16;
+      scale = (kLinear ? quad * g.a_row * kDdrWord : 0u) + 128;
+      shift = 8 * (r & 3);
     }
-    st.sa = aw[o.a_scale & 0xFFFFu];
-    LoadDwords<T::kW4>(ww + (o.w & 0xFFFFu), st.w);
-    st.sw = ww[o.w_scale & 0xFFFFu];
+  }
+};
+
+// Loads the thread's unit of a stage.
+template <bool kLinear, class T>
+__device__ __forceinline__ void LoadStage(const GemmArgs& g, const uint8_t* a, const uint8_t* w0,
+                                          const uint8_t* w1, const Lane<kLinear, T>& ln,
+                                          const Stage& s, Staged& st) {
+  const uint32_t last = max(s.live, 1u) - 1, blk = s.blk + min(ln.block, last);
+  const uint8_t* base = ln.w ? (s.l ? w1 : w0) : a;
+  if (kLinear) {
+    const uint32_t at = (blk >> ln.half) * ln.chunk, odd = blk & ln.half;
+    st.v = *reinterpret_cast<const u32x4*>(base + (size_t)(ln.codes + at + odd * ln.c_step));
+    st.scale = *reinterpret_cast<const uint32_t*>(base + (size_t)(ln.scale + at + odd * ln.s_step));
+  } else if (ln.w) {
+    const uint8_t* word = WWord<false>(g, base, ln.line, blk);
+    st.v = *reinterpret_cast<const u32x4*>(word + ln.codes);
+    st.scale = *reinterpret_cast<const uint32_t*>(word + ln.scale);
+  } else {  // ISS ABUF words are 132 B: only 4-byte aligned
+    const uint8_t* word = AWord<false>(g, base, ln.line, blk);
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(word + ln.codes);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) st.v[k] = src[k];
+    st.scale = *reinterpret_cast<const uint32_t*>(word + ln.scale);
   }
 }
 
-// 4 int8 -> 4 bf16 (2 dwords) scaled by fa = 2^(ea-127), exactly:
-// (2^23 + q + 128) * fa - (2^23 + 128) * fa = q * fa, one rounding of an
-// exact value.  The byte lands in a float's mantissa by v_perm_b32.
-__device__ __forceinline__ void ConvertA4(uint32_t x, float fa, float fc, uint32_t* out) {
-  const uint32_t xs = x ^ 0x80808080u;
-  float f[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    f[i] = __builtin_fmaf(__uint_as_float(__builtin_amdgcn_perm(0x4B000000u, xs, 0x070C0C00u | i)),
-                          fa, fc);
-  out[0] = __builtin_amdgcn_perm(__float_as_uint(f[1]), __float_as_uint(f[0]), 0x07060302u);
-  out[1] = __builtin_amdgcn_perm(__float_as_uint(f[3]), __float_as_uint(f[2]), 0x07060302u);
+// A byte n under the f16 exponent byte 0x64 is exactly 1024 + n.
+// perm(0x64646464, x, Sel(i, j)) is the f16 pair {1024 + byte i, 1024 + byte j}.
+constexpr uint32_t Sel(uint32_t i, uint32_t j) { return 0x04000400u | i | (j << 16); }
+__device__ __forceinline__ f16x2 Pair(uint32_t x, uint32_t sel) {
+  return __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, x, sel));
 }
+__device__ __forceinline__ uint32_t Bits(f16x2 v) { return __builtin_bit_cast(uint32_t, v); }
 
-// bf16 bits of a small integer (exact).
-__device__ __forceinline__ uint32_t Bf16OfInt(int32_t v) { return __float_as_uint((float)v) >> 16; }
+// What a staging thread has seen: a scale byte outside the window the
+// matrix-core path is exact for, or a row whose ea lies outside f16's.
+struct Seen {
+  bool unsafe = false, wide = false;
+};
 
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-
-// 8 FP4 codes (one dword, low nibble first) -> 8 bf16 of 2 * E2M1 value,
-// i.e. the reference's FP4 weight integers {0, +-1, ..., +-12}: one
-// v_cvt_scalef32_pk_bf16_fp4 per byte (scale 2.0, exact).
-__device__ __forceinline__ void ConvertFp4(uint32_t x, uint32_t* out) {
-  out[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(x, 2.0f, 0));
-  out[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(x, 2.0f, 1));
-  out[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(x, 2.0f, 2));
-  out[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(x, 2.0f, 3));
-}
-
-// Stage one block into LDS: A scaled to bf16, W as unscaled bf16 weight
-// integers, W scale bytes.  True if a scale byte is outside the window the
-// matrix-core path is exact for.
-template <class T, class S>
-__device__ __forceinline__ bool StoreBlock(const S& st, const Lane<T>& ln, uint32_t mode,
-                                           uint16_t* lds_a, uint16_t* lds_w, uint8_t* lds_ws,
-                                           const uint32_t* lut) {
-  const float fa = __uint_as_float(st.sa << 23);
-  const float fc = -8388736.0f * fa;  // -(2^23 + 128) * fa
-  uint32_t ab[2 * T::kA4];
+// Converts a stage into LDS buffer `buf`: A scaled to f16, W as unscaled f16
+// weight integers (FP4 codes by v_cvt_scalef32_pk_f16_fp4, nibbles by the
+// perm above), and the scale factors.  A W8 byte holds two K positions, so a
+// W8 block's elements come out in the order 0,2,1,3 of each 4; A is staged in
+// the same order for it (a block's sum does not depend on the order).
+template <int kFmt, bool kLinear, class T>
+__device__ __forceinline__ void StoreStage(const GemmArgs& g, const Lane<kLinear, T>& ln,
+                                           const Stage& s, const Staged& st, Lds<T>& lds,
+                                           uint32_t buf, Seen& seen) {
+  // the plane's mode (a W8 layer's planes are hi, lo)
+  const uint32_t mode = kFmt == kFmtFp4  ? (uint32_t)kModeFp4
+                        : kFmt == kFmtW8 ? (s.l ? (uint32_t)kModeW8Lo : (uint32_t)kModeW8Hi)
+                                         : (s.l ? g.modes[1] : g.modes[0]);
+  const bool fp4 = mode == kModeFp4;
+  const uint32_t e = __builtin_amdgcn_ubfe(st.scale, ln.shift, 8);
+  seen.unsafe |= e - kSafeLo > kSafeHi - kSafeLo;
+  if (!ln.w) {
+    if (T::kAUnits < 256 && (threadIdx.x & 255u) >= (uint32_t)T::kAUnits) return;
+    const uint32_t s01 = fp4 ? Sel(0, 1) : Sel(0, 2), s23 = fp4 ? Sel(2, 3) : Sel(1, 3);
+    const uint32_t r = ln.u / 2 % T::kBM, h = ln.u % 2;
+    const int32_t d = min(max((int32_t)e - kAUnit, kAMin), kAMax);
+    // f16 2^d and -1152 * 2^d: fma(1024 + q + 128, 2^d, -1152 * 2^d) = q * 2^d
+    const uint32_t live = ln.block < s.live ? 0xFFFFFFFFu : 0u;
+    const uint32_t d2 = __umul24((uint32_t)(d + 15), 0x000400u) * 0x00010001u;
+    const f16x2 f = __builtin_bit_cast(f16x2, d2 & live);
+    const f16x2 c = __builtin_bit_cast(f16x2, ((d2 + 0x28002800u) | 0x80808080u) & live);
+    uint32_t o[8];
 #pragma unroll
-  for (int i = 0; i < T::kA4; ++i) ConvertA4(st.a[i], fa, fc, ab + 2 * i);
-#pragma unroll
-  for (int i = 0; i < 2 * T::kA4; ++i) ab[i] = st.zero_a ? 0u : ab[i];
-  uint32_t* da = reinterpret_cast<uint32_t*>(lds_a + ln.r * kLdsRow + ln.aofs);
-  if (T::kA4 == 4) {
-    reinterpret_cast<u32x4*>(da)[0] = u32x4{ab[0], ab[1], ab[2], ab[3]};
-    reinterpret_cast<u32x4*>(da)[1] = u32x4{ab[4], ab[5], ab[6], ab[7]};
+    for (int k = 0; k < 4; ++k) {
+      const uint32_t x = st.v[k] ^ 0x80808080u;
+      o[2 * k] = Bits(__builtin_elementwise_fma(Pair(x, s01), f, c));
+      o[2 * k + 1] = Bits(__builtin_elementwise_fma(Pair(x, s23), f, c));
+    }
+    uint4* tile = lds.a[buf][ln.block][r / 16];
+    tile[Slot(2 * h, r % 16)] = uint4{o[0], o[1], o[2], o[3]};
+    tile[Slot(2 * h + 1, r % 16)] = uint4{o[4], o[5], o[6], o[7]};
+    const int32_t rest = (int32_t)e - kAUnit - d;
+    lds.fr[buf][ln.block][r] = __uint_as_float((uint32_t)(rest + 127) << 23);
+    seen.wide |= rest != 0;
   } else {
-    reinterpret_cast<u32x2*>(da)[0] = u32x2{ab[0], ab[1]};
+    if (T::kWUnits < 256 && (threadIdx.x & 255u) >= (uint32_t)T::kWUnits) return;
+    const uint32_t col = ln.u % T::kBN;
+    uint4* tile = lds.w[buf][ln.block][col / 16];
+    if (fp4) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t v = st.v[k];
+        tile[Slot(k, col % 16)] =
+            uint4{Bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, 2.0f, 0)),
+                  Bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, 2.0f, 1)),
+                  Bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, 2.0f, 2)),
+                  Bits(__builtin_amdgcn_cvt_scalef32_pk_f16_fp4(v, 2.0f, 3))};
+      }
+    } else {
+      const uint32_t flip = mode == kModeW8Hi ? 0x88888888u : 0u;
+      const _Float16 bias = mode == kModeW8Hi ? (_Float16)1032.0f : (_Float16)1024.0f;
+      const f16x2 sub = {bias, bias};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t v = st.v[k] ^ flip;
+        const uint32_t ev = v & 0x0F0F0F0Fu, od = (v >> 4) & 0x0F0F0F0Fu;
+        tile[Slot(k, col % 16)] =
+            uint4{Bits(Pair(ev, Sel(0, 1)) - sub), Bits(Pair(od, Sel(0, 1)) - sub),
+                  Bits(Pair(ev, Sel(2, 3)) - sub), Bits(Pair(od, Sel(2, 3)) - sub)};
+      }
+    }
+    lds.fw[buf][ln.block][col] =
+        __uint_as_float((uint32_t)((int32_t)e + ScaleBias(mode) + kAUnit - 127) << 23);
   }
-  uint32_t wb[4 * T::kW4];
-  if (mode == kModeFp4) {
-#pragma unroll
-    for (int i = 0; i < T::kW4; ++i) ConvertFp4(st.w[i], wb + 4 * i);
-  } else {
-    const uint32_t* tab = lut + st.plane * 256;
-#pragma unroll
-    for (int i = 0; i < T::kW4; ++i)
-#pragma unroll
-      for (int m = 0; m < 4; ++m) wb[4 * i + m] = tab[(st.w[i] >> (8 * m)) & 0xFFu];
-  }
-  u32x4* dw = reinterpret_cast<u32x4*>(lds_w + ln.col * kLdsRow + ln.wofs * 2);
-#pragma unroll
-  for (int i = 0; i < T::kW4; ++i) dw[i] = u32x4{wb[4 * i], wb[4 * i + 1], wb[4 * i + 2], wb[4 * i + 3]};
-  lds_ws[ln.col] = (uint8_t)st.sw;  // both threads of a column store the same byte
-  return st.sa < kSafeLo || st.sa > kSafeHi || st.sw < kSafeLo || st.sw > kSafeHi;
 }
 
 // Exact integer recomputation of one output (the NPU's arithmetic verbatim).
@@ -316,21 +338,33 @@ __device__ __forceinline__ uint32_t SlowOutput(const GemmArgs& g, const uint8_t*
   return acc;
 }
 
-// The exact tile kernel.  Per K block: stage A (bf16, scaled) and W (bf16,
-// unscaled) in LDS; per 16x16 tile one MFMA with a zero accumulator gives
-// s * 2^(ea-127) exactly; the fold is acc = fma(that, 2^(ew-127+SBIAS), acc),
-// a single rounding of an exact sum, which is the NPU's Fp32Add.  Operand
-// loads run a chunk of kChunk blocks ahead of the compute.
-template <bool kLinear, int kBM, int kBN>
-__global__ __launch_bounds__(kThreads) void GemmTileKernel(GemmArgs g) {
-  using T = Tile<kBM, kBN>;
-  using S = Staged<T::kA4, T::kW4>;
-  __shared__ __attribute__((aligned(16))) uint16_t lds_a[2][kBM * kLdsRow];
-  __shared__ __attribute__((aligned(16))) uint16_t lds_w[2][kBN * kLdsRow];
-  __shared__ __attribute__((aligned(16))) uint8_t lds_ws[2][kBN];
-  __shared__ uint32_t lut[2 * 256];
-  __shared__ uint64_t lds_act[512];  // activation half of TBUF, for the epilogue
-  __shared__ uint32_t lds_unsafe;
+// The exact tile kernel.  A stage is kC K blocks; while a stage is folded,
+// the raw bytes of the next two are on their way into registers; the next one
+// is converted into the other LDS buffer: one barrier per stage.  Per block
+// and 16x16 tile one MFMA with a zero accumulator gives s * 2^d exactly, and
+// the fold is an fma per output.
+//
+// Bound: the VALU beside the matrix cores.  A 16x16x32 MFMA takes 16.5
+// cycles and the 4 folds of its outputs as long; both together 23.3 where 3
+// waves of a SIMD take turns, 24.2 with 2, 37 with one (measured), so tiles
+// leave room for 2 or 3 workgroups per CU.  The rest is conversion: 5
+// instructions per 4 activations (an xor, two byte permutes, two packed f16
+// fmas; with bf16 operands, which have no packed arithmetic, it was 11) and
+// one per 2 FP4 weights.
+//
+// Measured, one launch: 4512 x 960, K 2560, MXFP4 with the residual 129 -> 56
+// us; 2048 x 2304, K 768, W8 with MULP and ADDP 111 -> 45 us (bf16 operands,
+// 128 x 128 tiles of 4 waves, one block a barrier, and the ops in integers
+// before). The K loop now takes about 1.6 times its VALU and matrix-core
+// cycles; the LDS moves 65 KB per 64 x 96 tile and stage, 0.6 of its rate.
+//
+// The loop runs with the rows' factors fr left out, which are 1 for every
+// ea in [116, 135]; every kCheck stages it looks whether a row had another,
+// and then starts again with them.
+template <bool kLinear, bool kMulti, int kFmt, class T>
+__global__ __launch_bounds__(kThreads, T::kWavesPerSimd) void GemmTileKernel(GemmArgs g) {
+  constexpr int kBM = T::kBM, kBN = T::kBN, kC = T::kC;
+  __shared__ __attribute__((aligned(16))) Lds<T> lds;
 
   const uint8_t* a = g.a;
   const uint8_t* w0 = g.w[0];
@@ -353,238 +387,209 @@ __global__ __launch_bounds__(kThreads) void GemmTileKernel(GemmArgs g) {
   const uint32_t q0 = tile.y * (kBM / 4), g0 = tile.x * (kBN / 8);
   const uint32_t row0 = q0 * 4, col0 = g0 * 8;
 
-  const Lane<T> ln;
-  const Offsets offs = ThreadOffsets<kLinear, T>(g, ln, q0, g0);
-  if (tid == 0) lds_unsafe = 0;
-  // byte -> two unscaled bf16 weight values (low nibble first), per plane
-  for (uint32_t l = 0; l < g.n_planes; ++l) {
-    const uint32_t mode = g.modes[l];
-    lut[l * 256 + tid] = Bf16OfInt(WeightValue(tid & 15u, mode)) |
-                         (Bf16OfInt(WeightValue(tid >> 4, mode)) << 16);
-  }
-  __syncthreads();  // the table and the cleared flag are visible to every wave
+  const Lane<kLinear, T> ln(g, q0, g0);
+  if (tid == 0) lds.unsafe = lds.wide = 0;
 
   // Output (i, j, v) of this lane: tile row wm*kTM + i*16 + kq*4 + v,
   // tile column wn*kTN + j*16 + row16 (16x16 MFMA accumulator layout).
   f32x4 acc[T::kTI][T::kTJ];
-  bool unsafe = false;
+  Seen seen;
+  auto start = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < T::kTI; ++i)
+#pragma unroll
+      for (int j = 0; j < T::kTJ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (!g.acc) return;
+#pragma unroll
+    for (int i = 0; i < T::kTI; ++i)
+#pragma unroll
+      for (int j = 0; j < T::kTJ; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const uint32_t row = row0 + wm * T::kTM + i * 16 + kq * 4 + v;
+          const uint32_t col = col0 + wn * T::kTN + j * 16 + row16;
+          const bool in = (row >> 2) < g.quads && (col >> 3) < g.groups && (!kLinear || row < g.m);
+          const uint32_t init = in ? *CElem<kLinear>(g, c, row, col) : 0u;
+          seen.unsafe |= ExpField(init) > 252u;
+          acc[i][j][v] = __uint_as_float(init);
+        }
+  };
+
+  const uint32_t stages = StageCount<kC>(g);
+  struct Operands {
+    f16x8 a[T::kTI], w[T::kTJ];
+    float fw[T::kTJ];
+  };
+  auto read = [&](uint32_t buf, int b, Operands& o) __attribute__((always_inline)) {
+    const uint32_t slot = Slot(kq, row16);
+#pragma unroll
+    for (int j = 0; j < T::kTJ; ++j) {
+      o.w[j] = __builtin_bit_cast(f16x8, lds.w[buf][b][wn * T::kTJ + j][slot]);
+      o.fw[j] = lds.fw[buf][b][wn * T::kTN + j * 16 + row16];
+    }
+#pragma unroll
+    for (int i = 0; i < T::kTI; ++i)
+      o.a[i] = __builtin_bit_cast(f16x8, lds.a[buf][b][wm * T::kTI + i][slot]);
+  };
+  // The fold of one stage; kWide: with the rows' own factors.
+  auto fold = [&](uint32_t buf, auto wide) __attribute__((always_inline)) {
+    constexpr bool kWide = decltype(wide)::value;
+#pragma unroll
+    for (int b = 0; b < kC; ++b) {
+      Operands x;
+      read(buf, b, x);
+#pragma unroll
+      for (int i = 0; i < T::kTI; ++i) {
+        f32x4 fr, bv[T::kTJ];
+        if (kWide)
+          fr = *reinterpret_cast<const f32x4*>(&lds.fr[buf][b][wm * T::kTM + i * 16 + kq * 4]);
+#pragma unroll
+        for (int j = 0; j < T::kTJ; ++j) {
+          const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+          bv[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x.a[i], x.w[j], zero, 0, 0, 0);
+        }
+#pragma unroll
+        for (int j = 0; j < T::kTJ; ++j) {
+          if (kWide) bv[j] = bv[j] * fr;
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            acc[i][j][v] = __builtin_fmaf(bv[j][v], x.fw[j], acc[i][j][v]);
+        }
+      }
+      // Anchor the fold here: left free, the compiler sinks every block's
+      // (pure) folds to the end of the stage, keeping all the blocks'
+      // values live at once.  The empty asm emits no instruction.
+#pragma unroll
+      for (int i = 0; i < T::kTI; ++i)
+#pragma unroll
+        for (int j = 0; j < T::kTJ; ++j) asm volatile("" : "+v"(acc[i][j]));
+      if (b + 1 < kC) __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // The whole fold; false if it met a row that needs its factor (without
+  // kWide).  Two stages a round, without a branch between the loads and their
+  // use, so that the loads of two stages stay in flight across the barriers.
+  auto run = [&](auto wide) __attribute__((always_inline)) {
+    constexpr bool kWide = decltype(wide)::value;
+    Cursor<kMulti, kC> cursor;
+    Stage cur[2];
+    Staged raw[2];
+    auto load = [&](int i) __attribute__((always_inline)) {
+      cur[i] = cursor.Take(g);
+      LoadStage<kLinear, T>(g, a, w0, w1, ln, cur[i], raw[i]);
+    };
+    auto store = [&](int i, uint32_t buf) __attribute__((always_inline)) {
+      StoreStage<kFmt, kLinear, T>(g, ln, cur[i], raw[i], lds, buf, seen);
+    };
+    load(0);
+    load(1);
+    start();
+    store(0, 0);
+    load(0);
+    __syncthreads();
+    for (uint32_t s = 0; s + 1 < stages; s += 2) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        fold(i, wide);
+        store(1 - i, 1 - i);
+        load(1 - i);
+        if (!kWide && i == 1 && seen.wide && s % kCheck == 0) lds.wide = 1;
+        __syncthreads();
+      }
+      // (uniform: the flag was raised before the barrier, and every wave is
+      // past the next one before it can be raised again)
+      if (!kWide && s % kCheck == 0 && __builtin_amdgcn_readfirstlane(lds.wide) != 0) return false;
+    }
+    if (stages & 1) fold(0, wide);
+    if (!kWide && seen.wide) lds.wide = 1;
+    __syncthreads();
+    return kWide || __builtin_amdgcn_readfirstlane(lds.wide) == 0;
+  };
+  if (!run(std::false_type{})) run(std::true_type{});
+  if (seen.unsafe) lds.unsafe = 1;
+  if (kLinear && g.tbuf != nullptr)
+    for (uint32_t i = tid; i < 512; i += kThreads) lds.act[i] = g.tbuf[512 + i];
+  // The outputs meet row by row in the staging buffers, -0 as +0.
 #pragma unroll
   for (int i = 0; i < T::kTI; ++i)
 #pragma unroll
     for (int j = 0; j < T::kTJ; ++j)
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const uint32_t row = row0 + wm * T::kTM + i * 16 + kq * 4 + v;
-        const uint32_t col = col0 + wn * T::kTN + j * 16 + row16;
-        uint32_t init = 0;
-        if (g.acc && (row >> 2) < g.quads && (col >> 3) < g.groups && (!kLinear || row < g.m)) {
-          init = *CElem<kLinear>(g, c, row, col);
-          unsafe |= ExpField(init) > 252u;
-        }
-        acc[i][j][v] = __uint_as_float(init);
-      }
-
-  // The step loop is one basic block: every wave runs every step (surplus
-  // steps of the last iteration repeat the last block with A zeroed, adding
-  // +0), the load cursor advances by selects, and scale bytes outside the
-  // safe window are collected per thread and acted on once, after the loop.
-  const uint32_t total = g.total_steps;
-  Step ls{0, 0, 0};  // load cursor; stays on the last step once there
-  uint32_t loaded = 0;
-  // Loads issue in program order (the fences stop the scheduler from mixing
-  // the two register sets), so the in-order load counter lets each compute
-  // wait for exactly its own set.
-  auto load_chunk = [&](S* set) {
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int b = 0; b < kChunk; ++b) {
-      LoadBlock<kLinear, T>(g, a, w0, w1, offs, ls, set[b]);
-      set[b].zero_a = loaded >= total;
-      const Step nx = Next(ls, g);
-      const bool adv = loaded + 1 < total;
-      ls.p = adv ? nx.p : ls.p;
-      ls.l = adv ? nx.l : ls.l;
-      ls.b = adv ? nx.b : ls.b;
-      ++loaded;
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  auto compute_chunk = [&](const S* set, uint32_t base) {
-#pragma unroll
-    for (int b = 0; b < kChunk; ++b) {
-      const uint32_t buf = (base + b) & 1;
-      unsafe |= StoreBlock<T>(set[b], ln, g.modes[set[b].plane], lds_a[buf], lds_w[buf],
-                              lds_ws[buf], lut);
-      __syncthreads();
-      const int32_t wbias = ScaleBias(g.modes[set[b].plane]);
-      bf16x8 af[T::kTI], bfr[T::kTJ];
-      float fw[T::kTJ];
-#pragma unroll
-      for (int i = 0; i < T::kTI; ++i)
-        af[i] = *reinterpret_cast<const bf16x8*>(
-            &lds_a[buf][(wm * T::kTM + i * 16 + row16) * kLdsRow + kq * 8]);
-#pragma unroll
-      for (int j = 0; j < T::kTJ; ++j) {
-        const uint32_t lc = wn * T::kTN + j * 16 + row16;
-        bfr[j] = *reinterpret_cast<const bf16x8*>(&lds_w[buf][lc * kLdsRow + kq * 8]);
-        fw[j] = __uint_as_float((uint32_t)((int32_t)lds_ws[buf][lc] + wbias) << 23);
-      }
-#pragma unroll
-      for (int i = 0; i < T::kTI; ++i)
-#pragma unroll
-        for (int j = 0; j < T::kTJ; ++j) {
-          const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-          const f32x4 bv = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bfr[j], zero, 0, 0, 0);
-#pragma unroll
-          for (int v = 0; v < 4; ++v) acc[i][j][v] = __builtin_fmaf(bv[v], fw[j], acc[i][j][v]);
-        }
-      // Anchor the fold here: left free, the compiler sinks every step's
-      // (pure) folds to the end of the iteration, keeping all the steps'
-      // block values live at once.  The empty asm emits no instruction.
-#pragma unroll
-      for (int i = 0; i < T::kTI; ++i)
-#pragma unroll
-        for (int j = 0; j < T::kTJ; ++j) asm volatile("" : "+v"(acc[i][j]));
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
-  // Ping-pong over two register sets: each compute consumes one set while
-  // the other set's loads are in flight.
-  S set0[kChunk], set1[kChunk];
-  load_chunk(set0);
-  for (uint32_t base = 0; base < total; base += 2 * kChunk) {
-    load_chunk(set1);
-    compute_chunk(set0, base);
-    load_chunk(set0);
-    compute_chunk(set1, base + kChunk);
-  }
-  if (unsafe) lds_unsafe = 1;
-  if (kLinear && g.tbuf != nullptr)
-    for (uint32_t i = tid; i < 512; i += kThreads) lds_act[i] = g.tbuf[512 + i];
+      for (int v = 0; v < 4; ++v)
+        lds.out[(wm * T::kTM + i * 16 + kq * 4 + v) * T::kOutRow + wn * T::kTN + j * 16 + row16] =
+            acc[i][j][v] + 0.0f;
   __syncthreads();
-  const bool slow = lds_unsafe != 0;
+  const bool slow = lds.unsafe != 0;
 
-  // Results as FP32 bits in one 16-value register vector per row tile i
-  // (element e = 4 * j + v).  i is unrolled and e, where a loop over it is
-  // not, is a wave-uniform index into the vector, so nothing goes through
-  // scratch memory.  The slow path recomputes the whole tile exactly.
-  static_assert(T::kTJ == 4, "four 16-column tiles per wave");
-  f32x16 res[T::kTI];
-#pragma unroll
-  for (int i = 0; i < T::kTI; ++i) {
-    const f32x8 lo = __builtin_shufflevector(acc[i][0], acc[i][1], 0, 1, 2, 3, 4, 5, 6, 7);
-    const f32x8 hi = __builtin_shufflevector(acc[i][2], acc[i][3], 0, 1, 2, 3, 4, 5, 6, 7);
-    res[i] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const uint32_t bits = __float_as_uint(res[i][e]);
-      res[i][e] = __uint_as_float(bits == kSign ? 0u : bits);
-    }
-  }
-  const uint32_t row_l = row0 + wm * T::kTM + kq * 4;
-  const uint32_t col_l = col0 + wn * T::kTN + row16;
-  if (slow) {
-#pragma unroll
-    for (int i = 0; i < T::kTI; ++i)
-      for (uint32_t e = 0; e < 16; ++e) {
-        const uint32_t row = row_l + i * 16 + (e & 3), col = col_l + (e >> 2) * 16;
-        if ((row >> 2) >= g.quads || (col >> 3) >= g.groups) continue;
+  // Epilogue: 4 consecutive columns of a row per thread and round, the ops
+  // in order, C as 16-byte stores; a row's 32-column block is 8 consecutive
+  // lanes, whose largest exponent field meets in three register moves.
+  const uint32_t rows4 = g.quads * 4, n = g.groups * 8;
+  const bool c16 = (reinterpret_cast<uintptr_t>(c) & 15u) == 0;  // uniform
+  constexpr uint32_t kUnits = kBM * kBN / 4;
+#pragma unroll 1
+  for (uint32_t u = tid; u < kUnits; u += kThreads) {
+    const uint32_t r = u / (kBN / 4), cc = u % (kBN / 4) * 4;
+    const uint32_t row = row0 + r, col = col0 + cc;
+    const bool in = row < rows4 && col < n;
+    f32x4 y = *reinterpret_cast<const f32x4*>(&lds.out[r * T::kOutRow + cc]);
+    if (slow && in) {  // the tile exactly
+#pragma unroll 1
+      for (uint32_t k = 0; k < 4; ++k) {
         uint32_t init = 0;
-        if (g.acc && (!kLinear || row < g.m)) init = *CElem<kLinear>(g, c, row, col);
-        res[i][e] = __uint_as_float(SlowOutput<kLinear>(g, a, w0, w1, init, row, col));
+        if (g.acc && (!kLinear || row < g.m)) init = *CElem<kLinear>(g, c, row, col + k);
+        y[k] = __uint_as_float(SlowOutput<kLinear>(g, a, w0, w1, init, row, col + k));
       }
-  }
-  if (kLinear && g.ws != nullptr) {  // deferred epilogue: the fold results, rows [0, 4*quads)
+    }
+    if (kLinear) {
+      for (uint32_t o = 0; o < g.n_ops; ++o) {
+        const uint32_t kind = g.op_kind[o];
+        f32x4 x2 = {0.f, 0.f, 0.f, 0.f}, p = x2;
+        if ((kind == kEpAdd || kind == kEpActMul) && in && row < g.m) {
+          const uint32_t* v = g.op_x2[o] + z * g.op_x2_batch[o] + (size_t)row * g.n + col;
+          if ((reinterpret_cast<uintptr_t>(g.op_x2[o] + z * g.op_x2_batch[o]) & 15u) == 0 &&
+              g.n % 4 == 0) {
+            x2 = *reinterpret_cast<const f32x4*>(v);
+          } else {
 #pragma unroll
-    for (int i = 0; i < T::kTI; ++i)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const uint32_t row = row_l + i * 16 + (e & 3), col = col_l + (e >> 2) * 16;
-        if ((row >> 2) < g.quads && (col >> 3) < g.groups) g.ws[(size_t)row * g.n + col] = res[i][e];
-      }
-    return;
-  }
-
-  // Epilogue ops, op by op, in groups of two row tiles.  A group's operands
-  // are loaded first, all at once (independent loads, one wait); the element
-  // loop then only computes.
-  if (kLinear) {
-    constexpr int kGroup = T::kTI >= 2 ? 2 : 1;
-    for (uint32_t o = 0; o < g.n_ops; ++o) {
-      const uint32_t kind = g.op_kind[o], imm = g.op_imm[o];
-      const bool has_x2 = kind == kEpAdd || kind == kEpActMul;
-      const uint32_t* x2 = g.op_x2[o] + z * g.op_x2_batch[o];
-      uint32_t pv[4] = {0u, 0u, 0u, 0u};
-      if (kind == kEpAddP || kind == kEpMulP) {
-        const uint32_t* v = g.op_vec[o] + z * g.op_vec_batch[o];
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) pv[jj] = col_l + jj * 16 < g.n ? v[col_l + jj * 16] : 0u;
-      }
-#pragma unroll
-      for (int i0 = 0; i0 < T::kTI; i0 += kGroup) {
-        f32x16 xv[kGroup] = {};
-        if (has_x2) {
-#pragma unroll
-          for (int ii = 0; ii < kGroup; ++ii)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-              const uint32_t row = row_l + (i0 + ii) * 16 + (e & 3), col = col_l + (e >> 2) * 16;
-              xv[ii][e] = __uint_as_float(row < g.m && col < g.n ? x2[(size_t)row * g.n + col] : 0u);
-            }
-        }
-#pragma unroll
-        for (int ii = 0; ii < kGroup; ++ii) {
-          const int i = i0 + ii;
-          for (uint32_t e = 0; e < 16; ++e) {
-            const uint32_t row = row_l + i * 16 + (e & 3), col = col_l + (e >> 2) * 16;
-            if ((row >> 2) < g.quads && (col >> 3) < g.groups)
-              res[i][e] = __uint_as_float(EpApply(kind, imm, __float_as_uint(res[i][e]),
-                                                  __float_as_uint(xv[ii][e]), pv[e >> 2], lds_act));
+            for (int k = 0; k < 4; ++k) x2[k] = __uint_as_float(v[k]);
           }
         }
+        if ((kind == kEpAddP || kind == kEpMulP) && in) {
+          const uint32_t* v = g.op_vec[o] + z * g.op_vec_batch[o] + col;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) p[k] = __uint_as_float(v[k]);
+        }
+        EpApply4(kind, g.op_imm[o], y, x2, p, lds.act);
       }
     }
-  }
+    if (in && (!kLinear || (row < g.m && g.c != nullptr))) {
+      uint32_t* dst = CElem<kLinear>(g, c, row, col);
+      if (c16) {
+        *reinterpret_cast<f32x4*>(dst) = y;
+      } else {
 #pragma unroll
-  for (int i = 0; i < T::kTI; ++i)
-#pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const uint32_t row = row_l + i * 16 + (e & 3), col = col_l + (e >> 2) * 16;
-      const bool in_tile = (row >> 2) < g.quads && (col >> 3) < g.groups;
-      if (in_tile && (!kLinear || (row < g.m && g.c != nullptr)))
-        *CElem<kLinear>(g, c, row, col) = __float_as_uint(res[i][e]);
+        for (int k = 0; k < 4; ++k) dst[k] = __float_as_uint(y[k]);
+      }
     }
-
-  // MXINT8 requantize: one ABUF word per quad and 32 columns.  A quad is the
-  // 4 accumulator rows (v) of one lane group (kq); a 32-column block is two
-  // 16-column tiles (j, j+1) over the 16 lanes of the group.
-  if (kLinear && q_out != nullptr) {
-    const uint32_t nb = g.n >> 5;
+    if (kLinear && q_out != nullptr) {  // MXINT8 requantize (n % 32 == 0)
+      uint32_t e = 0;
 #pragma unroll
-    for (int i = 0; i < T::kTI; ++i) {
-      const uint32_t quad = q0 + (wm * T::kTM + i * 16) / 4 + kq;
+      for (int k = 0; k < 4; ++k) e = max(e, ExpField(__float_as_uint(y[k])));
+      e = max(e, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)e, 0xB1, 0xF, 0xF, false));
+      e = max(e, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)e, 0x4E, 0xF, 0xF, false));
+      e = max(e, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)e, 0x141, 0xF, 0xF, false));
+      if (in) {
+        uint8_t* word = q_out + ((size_t)(row >> 2) * (n >> 5) + (col >> 5)) * kDdrWord;
+        uint32_t codes = 0;
 #pragma unroll
-      for (int jb = 0; jb < T::kTJ; jb += 2) {
-        const uint32_t blk = (col0 + wn * T::kTN + jb * 16) >> 5;
-        uint32_t emax[4];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          emax[v] = RowMax16(max(ExpField(__float_as_uint(res[i][4 * jb + v])),
-                                 ExpField(__float_as_uint(res[i][4 * jb + 4 + v]))));
-        }
-        if (quad < g.quads && blk < nb) {
-          uint8_t* word = q_out + ((size_t)quad * nb + blk) * kDdrWord;
-#pragma unroll
-          for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-              word[v * 32 + jj * 16 + row16] =
-                  QuantizeElementHw(__float_as_uint(res[i][4 * (jb + jj) + v]), emax[v]);
-          const uint32_t e_own =
-              row16 == 0 ? emax[0] : row16 == 1 ? emax[1] : row16 == 2 ? emax[2] : emax[3];
-          if (row16 < 4) word[128 + row16] = (uint8_t)ScaleByteOf(e_own);
-          if (row16 >= 4) word[128 + row16] = 0;  // bytes 132..143
-        }
+        for (int k = 0; k < 4; ++k)
+          codes |= (uint32_t)QuantizeElementHw(__float_as_uint(y[k]), e) << (8 * k);
+        const uint32_t part = (col >> 2) & 7;
+        *reinterpret_cast<uint32_t*>(word + (row & 3) * 32 + part * 4) = codes;  // (4-aligned)
+        if (part == 0) word[128 + (row & 3)] = (uint8_t)ScaleByteOf(e);
+        if ((row & 3) == 0 && part >= 1 && part < 4)  // bytes 132..143
+          *reinterpret_cast<uint32_t*>(word + 128 + 4 * part) = 0u;
       }
     }
   }
@@ -630,34 +635,52 @@ __global__ __launch_bounds__(32) void GemmAliasKernel(GemmArgs g) {
 
 }  // namespace
 
-// 32 x 256 exact tiles for layers of at most 32 rows, and where the
-// 128 x 128 grid (with the batch) leaves CUs idle while 32 x 256 tiles make
-// more workgroups: each output's fold is sequential over K, so a small grid
-// is parallel only across tiles (measured: SigLIP's 2048 x 768 x 3072 W8
-// layer 235 -> 201 us, the SparseDrive-S head's layers at one frame 15-28%
-// faster).
-bool ExactShort(const GemmArgs& args, uint32_t batch) {
-  if (args.quads * 4 <= 32) return true;
-  const uint64_t tall = (uint64_t)((args.groups + 15) / 16) * ((args.quads + 31) / 32) * batch;
-  const uint64_t shrt = (uint64_t)((args.groups + 31) / 32) * ((args.quads + 7) / 8) * batch;
-  return tall < (uint64_t)DeviceCus() && shrt > tall;
-}
-
-template <bool kLinear>
-hipError_t LaunchTiles(const GemmArgs& in, uint32_t batch, hipStream_t stream) {
-  GemmArgs args = in;
+namespace {
+template <bool kLinear, class T>
+void LaunchTile(GemmArgs args, uint32_t batch, hipStream_t stream) {
   args.gz = batch;
-  if (!kLinear ? args.quads * 4 <= 32 : ExactShort(args, batch)) {
-    args.gx = (args.groups + 31) / 32;
-    args.gy = (args.quads + 7) / 8;
-    hipLaunchKernelGGL((GemmTileKernel<kLinear, 32, 256>), dim3(args.gx * args.gy * batch),
-                       dim3(kThreads), 0, stream, args);
+  args.gx = (args.groups * 8 + T::kBN - 1) / T::kBN;
+  args.gy = (args.quads * 4 + T::kBM - 1) / T::kBM;
+  const dim3 grid(args.gx * args.gy * batch), block(kThreads);
+  if constexpr (!kLinear) {
+    hipLaunchKernelGGL((GemmTileKernel<false, false, kFmtAny, T>), grid, block, 0, stream, args);
   } else {
-    args.gx = (args.groups + 15) / 16;
-    args.gy = (args.quads + 31) / 32;
-    hipLaunchKernelGGL((GemmTileKernel<kLinear, 128, 128>), dim3(args.gx * args.gy * batch),
-                       dim3(kThreads), 0, stream, args);
+    const bool fp4 = args.n_planes == 1 && args.modes[0] == kModeFp4;
+    const bool w8 = args.n_planes == 2 && args.modes[0] == kModeW8Hi && args.modes[1] == kModeW8Lo;
+    if (args.n_pieces == 1 && fp4)
+      hipLaunchKernelGGL((GemmTileKernel<true, false, kFmtFp4, T>), grid, block, 0, stream, args);
+    else if (args.n_pieces == 1 && w8)
+      hipLaunchKernelGGL((GemmTileKernel<true, false, kFmtW8, T>), grid, block, 0, stream, args);
+    else
+      hipLaunchKernelGGL((GemmTileKernel<true, true, kFmtAny, T>), grid, block, 0, stream, args);
   }
+}
+}  // namespace
+
+// The tile of a launch: the one with the least estimated time per K block, a
+// CU's tiles one after the other at the shape's rate, or one tile's latency.
+// Each output's fold is sequential over K, so a launch is parallel only over
+// its tiles: large tiles convert less per output, small ones fill the CUs.
+// The rates (ns per tile and block, and the least per block) are fitted to
+// these times, one launch each (us, 64x96 / 64x128 / 32x64):
+//   4512 x 960, K 2560    56 / 75 / 96     141 x 2560, K 960   17 / 20 / 11
+//   2048 x 2304, W8 768   45 / 55 / 67     141 x 960, K 2560   29 / 31 / 17
+//   2048 x 768, W8 768    27 / 26 / 26     1 x 960, K 960      13 / 13 / 9
+//   4512 x 320, K 960     25 / 21 / 22     928 x 512, W8 512   21 / 22 / 11
+//   32 layers of 128 x 960, K 2560   60 / 51 / 85
+template <bool kLinear>
+hipError_t LaunchTiles(const GemmArgs& args, uint32_t batch, hipStream_t stream) {
+  const uint64_t cus = DeviceCus(), cols = args.groups * 8ull, rows = args.quads * 4ull;
+  auto time = [&](uint64_t bm, uint64_t bn, uint64_t rate, uint64_t latency) {
+    const uint64_t tiles = ((rows + bm - 1) / bm) * ((cols + bn - 1) / bn) * batch;
+    const uint64_t t = (tiles + cus - 1) / cus * rate;
+    return t > latency ? t : latency;
+  };
+  const uint64_t t0 = time(32, 64, 130, 200), t1 = time(64, 96, 200, 400),
+                 t2 = time(64, 128, 260, 460);
+  if (t0 <= t1 && t0 <= t2) LaunchTile<kLinear, Tile<32, 64, 2, 4, 4>>(args, batch, stream);
+  else if (t1 <= t2) LaunchTile<kLinear, Tile<64, 96, 4, 2, 6>>(args, batch, stream);
+  else LaunchTile<kLinear, Tile<64, 128, 2, 2, 4>>(args, batch, stream);
   return hipGetLastError();
 }
 
@@ -672,21 +695,10 @@ hipError_t LaunchGemmInstrAliased(const GemmArgs& args, hipStream_t stream) {
   return hipGetLastError();
 }
 
-bool ExactShort(const GemmArgs& args, uint32_t batch);
-void ExactGrid(const GemmArgs& args, uint32_t* gx, uint32_t* gy) {
-  if (ExactShort(args, 1)) {
-    *gx = (args.groups + 31) / 32;
-    *gy = (args.quads + 7) / 8;
-  } else {
-    *gx = (args.groups + 15) / 16;
-    *gy = (args.quads + 31) / 32;
-  }
-}
-
 namespace {
-// A single layer with fewer tiles than this spreads its work: K splits in
-// fast mode (to about kTargetWorkgroups workgroups, at least kMinSplitSteps
-// K-steps each) and the element-parallel deferred epilogue.  Measured on the
+// A single fast layer with fewer tiles than this splits its K range (to
+// about kTargetWorkgroups workgroups, at least kMinSplitSteps K-steps each)
+// and finishes in the element-parallel deferred epilogue.  Measured on the
 // SmolVLA chains (M = 141 and 1,600): 128 workgroups of at least 4 steps beat
 // 256 of 2 by 9-13% (the split sums written and read again cost more than the
 // parallelism gains); 32 workgroups, or no split, lost 50-70% at M = 141.
@@ -804,9 +816,9 @@ hipError_t LaunchLinear(const GemmArgs& in, uint32_t batch, bool fast, Workspace
   // Batched layers of up to 16 rows: split-K over the waves of one
   // workgroup, which holds every row.
   if (fastk && args.quads * 4 <= 16) return LaunchLinearSkinny(args, batch, stream);
+  if (!fastk) return LaunchTiles<true>(args, batch, stream);
   uint32_t gx, gy;
-  if (fastk) FastGrid(args, batch, &gx, &gy, &args.tile_rows);
-  else ExactGrid(args, &gx, &gy);
+  FastGrid(args, batch, &gx, &gy, &args.tile_rows);
   args.gx = gx;
   args.gy = gy;
   const bool small = batch == 1 && gx * gy < kSmallGrid;
@@ -819,13 +831,13 @@ hipError_t LaunchLinear(const GemmArgs& in, uint32_t batch, bool fast, Workspace
   // even, 1024 x 2560 x 960 34.3 against 28.9 us).
   uint32_t blocks = 0;
   for (uint32_t p = 0; p < args.n_pieces; ++p) blocks += args.piece_kb[p];
-  if (small && fastk && args.quads * 4 <= kSplitMidRows &&
+  if (small && args.quads * 4 <= kSplitMidRows &&
       args.quads * 4 * blocks <= kSplitMidWork) {
     SplitPlan(args);
     args.fast_ep = 1u;
     return LaunchSplitLinear(args, stream);
   }
-  args.fast_ep = fastk ? 1u : 0u;
+  args.fast_ep = 1u;
   // Over panels the streaming kernel takes plain batched layers (and
   // MXFP8); a plain single layer takes the panel kernel, whose 8 waves per
   // CU hide more latency where a workgroup has one or two tiles (measured,
@@ -836,10 +848,10 @@ hipError_t LaunchLinear(const GemmArgs& in, uint32_t batch, bool fast, Workspace
   // streaming kernel's on 4 (measured on the SparseDrive backbone's layers,
   // e.g. 67,584 x 256 x 128 with bias, ReLU and the requantize: 55 against
   // 139 us).
-  if (fastk && !small && StreamEligible(args) && (batch > 1 || args.a_fp8))
+  if (!small && StreamEligible(args) && batch > 1)
     return LaunchStream(args, batch, stream);
-  if (fastk && !small && PanelEligible(args)) return LaunchPanel(args, batch, stream);
-  if (small && fastk) {
+  if (!small && PanelEligible(args)) return LaunchPanel(args, batch, stream);
+  if (small) {
     // as many splits as fit in one round of kTargetWorkgroups workgroups
     uint32_t nblocks = 0;
     for (uint32_t p = 0; p < args.n_pieces; ++p) nblocks += args.piece_kb[p];
@@ -850,10 +862,7 @@ hipError_t LaunchLinear(const GemmArgs& in, uint32_t batch, bool fast, Workspace
     args.splits = (steps + per - 1) / per;
     args.split_steps = per;
   }
-  // The exact kernels' epilogue arithmetic is spread over the elements of a
-  // small layer; the fast kernels finish an unsplit tile in place.
-  const bool defer = small && (args.splits > 1 || (!fastk && (args.n_ops > 0 || args.q_out != nullptr)));
-  if (!defer) return fastk ? LaunchLinearFast(args, batch, stream) : LaunchTiles<true>(args, batch, stream);
+  if (args.splits <= 1) return LaunchLinearFast(args, batch, stream);
 
   // (the partial sums start after the split counters)
   if (fixed != nullptr) {  // no allocation: the caller's buffer, or an error
@@ -865,8 +874,7 @@ hipError_t LaunchLinear(const GemmArgs& in, uint32_t batch, bool fast, Workspace
     if (grown != hipSuccess) return grown;
     args.ws = ws.ptr + kSplitCounterBytes / sizeof(float);
   }
-  const hipError_t err = fastk ? LaunchLinearFast(args, args.splits, stream)  // z = split
-                             : LaunchTiles<true>(args, 1, stream);
+  const hipError_t err = LaunchLinearFast(args, args.splits, stream);  // z = split
   if (err != hipSuccess) return err;
   return LaunchEpilogue(args, stream);
 }

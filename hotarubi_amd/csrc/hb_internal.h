@@ -241,9 +241,9 @@ uint32_t BandFor(uint32_t gx, uint32_t gy, uint64_t a_tile, uint64_t w_tile);
 // Launchers (hb_gemm.hip).
 hipError_t LaunchGemmInstr(const GemmArgs& args, hipStream_t stream);
 hipError_t LaunchGemmInstrAliased(const GemmArgs& args, hipStream_t stream);
-// Linear layer: picks the kernel, and for a single small layer (few tiles)
-// K splits (fast mode) and/or the deferred element-parallel epilogue, in
-// which case it may grow `ws` (GrowWorkspace).
+// Linear layer: picks the kernel, and for a single small fast layer (few
+// tiles) K splits and the deferred element-parallel epilogue, in which case
+// it may grow `ws` (GrowWorkspace).
 // A fixed scratch buffer in place of the context's growable workspace:
 // the launch never allocates; *need reports the bytes a layer needs.
 struct FixedScratch {
@@ -330,8 +330,6 @@ struct SplitGroup {
   uint32_t tile_end[kMaxGroup], first[kMaxGroup], second[kMaxGroup], x2_op[kMaxGroup];
 };
 hipError_t LaunchSplitGroup(const SplitGroup& grp, uint32_t waves, hipStream_t stream);
-// Exact tile kernel grid for a linear layer (column tiles, row tiles).
-void ExactGrid(const GemmArgs& args, uint32_t* gx, uint32_t* gy);
 // Deferred epilogue (hb_vec.hip): reads args.ws, writes C and q_out.
 hipError_t LaunchEpilogue(const GemmArgs& args, hipStream_t stream);
 

@@ -324,8 +324,8 @@ int hb_linear_group_async(hb_ctx* ctx, const hb_linear_desc* descs, uint32_t cou
  * the reference: it is for callers that cannot allocate device memory (code
  * under HIP graph capture, serving loops and harnesses that forbid
  * hipMalloc).  The partial sums and slow flags of a small layer's K splits
- * across workgroups (fast layers of more than 1,024 rows on few tiles, and
- * small exact layers with ops or requantize), which hb_linear keeps in the
+ * across workgroups (fast layers of more than 1,024 rows on few tiles),
+ * which hb_linear keeps in the
  * context's growable workspace, go to a fixed per-device scratch array of
  * HB_NOALLOC_SCRATCH_BYTES instead
  * (resolved when a context is created on the device, held until the
