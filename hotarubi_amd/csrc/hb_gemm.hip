@@ -817,6 +817,22 @@ hipError_t LaunchLinear(const GemmArgs& in, uint32_t batch, bool fast, Workspace
   // workgroup, which holds every row.
   if (fastk && args.quads * 4 <= 16) return LaunchLinearSkinny(args, batch, stream);
   if (!fastk) return LaunchTiles<true>(args, batch, stream);
+  // A batch of such layers whose 32 x 32 tiles are at most two to a CU:
+  // the split kernel's tiles too, where the tile kernel's 64-row tiles leave
+  // most CUs idle.  Measured, a launch (us, tile kernel / split tiles):
+  // 32 layers of 50 x 192, W8 K 64 (attention scores; 384 split tiles) 10.0
+  // / 5.5; 128 of 50 x 64, K 192 (512) 10.3 / 6.5; 16 of 64 x 320, K 960
+  // (320) 15.3 / 9.5; 4 of 128 x 960, K 2560 (480) 26.2 / 14.3; past two to
+  // a CU the larger tiles win: 128 of 50 x 192, K 64 (1,536) 10.6 / 13.9; 8
+  // of 141 x 960, K 960 (1,200) 16.0 / 22.4.
+  if (batch > 1 && args.quads * 4 <= kSplitMaxRows) {
+    GemmArgs split = args;
+    SplitPlan(split);
+    if ((uint64_t)split.gx * split.gy * batch <= 2ull * DeviceCus()) {
+      split.fast_ep = 1u;
+      return LaunchSplitBatch(split, batch, stream);
+    }
+  }
   uint32_t gx, gy;
   FastGrid(args, batch, &gx, &gy, &args.tile_rows);
   args.gx = gx;

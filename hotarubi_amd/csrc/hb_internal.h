@@ -312,6 +312,8 @@ constexpr uint32_t kMaxSplitWaves = 8;
 constexpr uint32_t kSplitFinishWaves = 4;
 size_t SplitPlan(GemmArgs& args, uint32_t max_splits = kMaxSplitWaves);
 hipError_t LaunchSplitLinear(const GemmArgs& args, hipStream_t stream);
+// The same tiles for `batch` layers (int8 activations; args from SplitPlan).
+hipError_t LaunchSplitBatch(const GemmArgs& args, uint32_t batch, hipStream_t stream);
 // Up to kMaxGroup single-launch split layers (args from SplitPlan, one
 // format) in one launch: units of one layer or a fused pair (the second's op
 // x2_op reads the first's C); second[u] == kMaxGroup for a single layer;

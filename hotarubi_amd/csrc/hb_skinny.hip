@@ -475,14 +475,24 @@ __device__ __forceinline__ SplitHot HotOf(const GemmArgs& g) {
 }
 
 // kSingle: the single-layer launch (its arguments untouched until its
-// loads are out; the epilogue's scalars pinned in SGPRs), else a group's.
-template <bool kW8, bool kMulti, bool kA8 = false, bool kSingle = false>
+// loads are out; the epilogue's scalars pinned in SGPRs), else a group's or
+// a batch's (z: the layer of the batch; h's pointers are that layer's).
+template <bool kW8, bool kMulti, bool kA8 = false, bool kSingle = false, bool kBatch = false>
 __device__ __forceinline__ void SplitTile(const GemmArgs& g, const SplitHot& h,
                                           uint32_t tile, uint32_t split,
                                           uint32_t nwaves, float (*lds_part)[16 * 64],
                                           uint32_t* lds_flag,
                                           bool pair, float* y_lds, const float* x2_lds,
-                                          uint32_t x2_op) {
+                                          uint32_t x2_op, uint32_t z = 0) {
+  // the layer's operands past A and W
+  auto g_c = [&] { return kBatch && g.c != nullptr ? g.c + z * g.c_batch : g.c; };
+  auto g_q = [&] { return kBatch && g.q_out != nullptr ? g.q_out + z * g.q_batch : g.q_out; };
+  auto g_vec = [&](uint32_t op) {
+    return kBatch ? g.op_vec[op] + z * g.op_vec_batch[op] : g.op_vec[op];
+  };
+  auto g_x2 = [&](uint32_t op) {
+    return kBatch ? g.op_x2[op] + z * g.op_x2_batch[op] : g.op_x2[op];
+  };
   constexpr int kWP = kW8 ? 2 : 1;
   typedef f32x16s f32x16;
   const uint32_t lane = threadIdx.x & 63;
@@ -684,17 +694,17 @@ __device__ __forceinline__ void SplitTile(const GemmArgs& g, const SplitHot& h,
     if (g.acc) {
 #pragma unroll
       for (int e = 0; e < 16; ++e)
-        if (owns(e)) pre_init[e] = __uint_as_float(g.c[crow(e)]);
+        if (owns(e)) pre_init[e] = __uint_as_float(g_c()[crow(e)]);
     }
 #pragma unroll
     for (int op = 0; op < kPreOps; ++op) {
       if ((uint32_t)op >= g.n_ops || (x2_lds && op == (int)x2_op)) continue;
       const uint32_t kind = g.op_kind[op];
-      if (kind == kEpAddP || kind == kEpMulP) pre_v[op] = __uint_as_float(g.op_vec[op][ccol]);
+      if (kind == kEpAddP || kind == kEpMulP) pre_v[op] = __uint_as_float(g_vec(op)[ccol]);
       if (kind == kEpAdd || kind == kEpActMul) {
 #pragma unroll
         for (int e = 0; e < 16; ++e)
-          if (owns(e)) pre_x2[op][e] = __uint_as_float(g.op_x2[op][crow(e)]);
+          if (owns(e)) pre_x2[op][e] = __uint_as_float(g_x2(op)[crow(e)]);
       }
     }
   }
@@ -711,8 +721,8 @@ __device__ __forceinline__ void SplitTile(const GemmArgs& g, const SplitHot& h,
   auto e_n = [&] { return kSingle ? p_n : g.n; };
   auto e_quads = [&] { return kSingle ? p_quads : g.quads; };
   auto e_ops = [&] { return kSingle ? p_ops : g.n_ops; };
-  auto e_c = [&] { return kSingle ? p_c : g.c; };
-  auto e_q = [&] { return kSingle ? p_q : g.q_out; };
+  auto e_c = [&] { return kSingle ? p_c : g_c(); };
+  auto e_q = [&] { return kSingle ? p_q : g_q(); };
   auto e_t = [&] { return kSingle ? p_t : g.tbuf; };
   bool slow = __builtin_amdgcn_ballot_w64(unsafe) != 0;
   f32x16 sum = acc;
@@ -786,12 +796,12 @@ __device__ __forceinline__ void SplitTile(const GemmArgs& g, const SplitHot& h,
             for (int i = 0; i < 4; ++i) x2[i] = row_of(4 * j + i) < e_m() ? pre_x2[o][4 * j + i] : 0.0f;
           }
       } else if (col_in) {
-        if (kind == kEpAddP || kind == kEpMulP) pv = __uint_as_float(g.op_vec[op][col]);
+        if (kind == kEpAddP || kind == kEpMulP) pv = __uint_as_float(g_vec(op)[col]);
         if (kind == kEpAdd || kind == kEpActMul) {
 #pragma unroll
           for (int i = 0; i < 4; ++i)
             if (row_of(4 * j + i) < e_m())
-              x2[i] = __uint_as_float(g.op_x2[op][(size_t)row_of(4 * j + i) * e_n() + col]);
+              x2[i] = __uint_as_float(g_x2(op)[(size_t)row_of(4 * j + i) * e_n() + col]);
         }
       }
       EpApplyFastN<false>(kind, g.op_imm[op], y, x2, pv, act);
@@ -855,6 +865,25 @@ __global__ __launch_bounds__(64 * kMaxSplitWaves) void SplitKernel(
   SplitTile<kW8, kMulti, kA8, true>(g, h, XcdLogical(blockIdx.x, tiles),
                          __builtin_amdgcn_readfirstlane(threadIdx.x >> 6),
                          blockDim.x / 64, lds_part, lds_flag, false, nullptr, nullptr, 0);
+}
+
+// A batch of layers of one shape, gx * gy workgroups to a layer (int8
+// activations): latency-bound like a single one, so a few layers share the
+// time of one launch.
+template <bool kW8, bool kMulti>
+__global__ __launch_bounds__(64 * kMaxSplitWaves) void SplitBatchKernel(GemmArgs g) {
+  __shared__ __attribute__((aligned(16))) float lds_part[kMaxSplitWaves][16 * 64];
+  __shared__ uint32_t lds_flag[kMaxSplitWaves];
+  TouchArgs(&g, sizeof g);
+  const uint32_t tiles = g.gx * g.gy, l = XcdLogical(blockIdx.x, gridDim.x), z = l / tiles;
+  SplitHot h = HotOf(g);
+  h.a += z * g.a_batch;
+  h.w0 += z * g.w_batch;
+  h.w1 += z * g.w_batch;
+  SplitTile<kW8, kMulti, false, false, true>(g, h, l % tiles,
+                                           __builtin_amdgcn_readfirstlane(threadIdx.x >> 6),
+                                           blockDim.x / 64, lds_part, lds_flag, false, nullptr,
+                                           nullptr, 0, z);
 }
 
 // A group of layers in one launch: unit u owns workgroups [tile_end[u - 1],
@@ -965,6 +994,19 @@ hipError_t LaunchSplitLinear(const GemmArgs& args, hipStream_t stream) {
     else hipLaunchKernelGGL((SplitKernel<false, false>), grid, block, 0, stream, HB_SPLIT_ARGS);
   }
 #undef HB_SPLIT_ARGS
+  return hipGetLastError();
+}
+
+hipError_t LaunchSplitBatch(const GemmArgs& args, uint32_t batch, hipStream_t stream) {
+  const dim3 grid(args.gx * args.gy * batch), block(64 * std::max(args.splits, kSplitFinishWaves));
+  const bool w8 = args.n_planes == 2, multi = args.n_pieces > 1;
+  if (w8) {
+    if (multi) hipLaunchKernelGGL((SplitBatchKernel<true, true>), grid, block, 0, stream, args);
+    else hipLaunchKernelGGL((SplitBatchKernel<true, false>), grid, block, 0, stream, args);
+  } else {
+    if (multi) hipLaunchKernelGGL((SplitBatchKernel<false, true>), grid, block, 0, stream, args);
+    else hipLaunchKernelGGL((SplitBatchKernel<false, false>), grid, block, 0, stream, args);
+  }
   return hipGetLastError();
 }
 
