@@ -5,14 +5,8 @@ and 4512 rows), LayerNorm at the SigLIP width (768), softmax over 141 of 192
 keys, fp32 and MXINT8 outputs, a last quad with fewer than 4 rows, and the
 argument checks.  The MXINT8 words feed hb_linear as its A.
 
-Every form of the kernel runs.  The library picks, per launch, the form
-with the fewest rounds of the CUs: the source rows kept in LDS or read again
-by each pass that takes them, 128, 256 or 1,024 threads per quad.  On a 256-CU
-MI355X: up to 512 quads (two per CU) run 1,024 threads with the rows kept
-(most cases here); RMSNorm 3001 x 960 (751 quads) runs 256 threads and
-softmax 24,960 x 192 128 threads with the rows kept; RMSNorm 4512 x 960 (1,128 quads, 4
-resident per CU with the rows kept and 6 without) and LayerNorm 6000 x 768
-(1,500 quads, 5 and 7) run 256 threads reading the rows again."""
+A row takes 64, 32 or 16 lanes by its width; quads with a row whose
+exponents leave the range of the plain FP32 passes run the guarded ones."""
 from __future__ import annotations
 
 import sys
@@ -136,6 +130,68 @@ def test_softmax_attention_rows(gpu, rows, cols, valid, quantize):
     tb = helpers.activation_table("silu")
     got = run_rows(gpu, 12, x, valid, tbuf=tb, quantize=quantize)
     check(got, oracle_rows(12, x, valid, 0, tbuf=tb, quantize=quantize))
+
+
+# Every lane layout (16, 32 or 64 lanes and up to 8 units of 4 columns a
+# lane; 24,960 x 192 above takes 16 lanes of 3) at its narrowest and widest,
+# row counts that leave a partial quad, wave and workgroup; ordinary rows and,
+# `special`, rows that need the guarded passes: every exponent, infinities
+# and NaN encodings, subnormals, zeros of both signs, constant rows, products
+# near 2^-126.
+@pytest.mark.parametrize("special", [False, True])
+@pytest.mark.parametrize("entry,cols", [
+    (34, 8), (34, 64), (34, 72), (34, 128), (34, 136), (34, 256), (34, 264), (34, 512), (34, 520),
+    (34, 768), (34, 1024), (34, 1032), (34, 1536), (34, 1544), (34, 2040), (22, 32), (22, 96),
+    (22, 224), (22, 544), (22, 960), (22, 1056), (22, 2016), (12, 40), (12, 64), (12, 128),
+    (12, 192), (12, 264), (12, 776), (12, 1544), (12, 2040)])
+def test_widths_and_special_rows(gpu, entry, cols, special):
+    rng = np.random.default_rng(entry * 10000 + cols + special)
+    rows = 61
+    x = activations(rng, rows, cols, 4.0)
+    aux = cols if entry != 12 or cols % 16 else cols - 5
+    gamma = helpers.random_fp32_words(rng, (cols,), 120, 130) if entry != 12 else None
+    beta = helpers.random_fp32_words(rng, (cols,), 110, 130) if entry == 22 else None
+    if special:
+        odd = helpers.random_fp32_words(rng, (rows, cols), 0, 255)
+        pick = rng.random((rows, cols)) < 0.01
+        pick[rng.random(rows) < 0.5] = False  # half of the rows stay ordinary
+        x[pick] = odd[pick]
+        x[5] = 0
+        x[6] = 0x80000000
+        x[7] = 0x3F800000  # constant: zero variance
+        x[8] = (np.float32(1e-20) * rng.standard_normal(cols).astype(np.float32)).view(np.uint32)
+        x[9] = (np.float32(1e25) * rng.standard_normal(cols).astype(np.float32)).view(np.uint32)
+        x[10, ::3] = 0x7F800000
+        x[11, ::2] = 0xFF800000  # a mask of infinities
+        x[12] = np.full(cols, -1e4, np.float32).view(np.uint32)
+        x[13] = np.linspace(-95.0, -60.0, cols).astype(np.float32).view(np.uint32)
+        x[13, 0] = 0  # exponentials down to 2^-126 and below
+        x[14] = 0xFF7FFFFF  # the type's lowest value everywhere
+        x[15] = 0xFF800000
+        if entry == 12 and aux < cols:
+            x[20:30, aux:] = 0x7FC00000  # NaN past the valid columns
+        if gamma is not None and cols > 512:
+            gamma[rng.random(cols) < 0.002] = 0x00000001  # (then every quad is guarded)
+    tb = helpers.activation_table("silu")
+    for quantize in ((False, True) if cols % 32 == 0 else (False,)):
+        got = run_rows(gpu, entry, x, aux, EPS, gamma=gamma, beta=beta, tbuf=tb, quantize=quantize)
+        check(got, oracle_rows(entry, x, aux, EPS, gamma=gamma, beta=beta, tbuf=tb,
+                               quantize=quantize))
+
+
+def test_rows_off_16_byte_boundaries(gpu):
+    rng = np.random.default_rng(3)
+    rows, cols = 30, 96
+    x = activations(rng, rows, cols)
+    gamma = helpers.random_fp32_words(rng, (cols,), 124, 128)
+    x_d = torch.zeros(rows * cols + 1, device=DEV)
+    g_d = torch.zeros(cols + 3, device=DEV)
+    y_d = torch.zeros(rows * cols + 2, device=DEV)
+    x_d[1:] = dev(x.view(np.float32)).view(-1)
+    g_d[3:] = dev(gamma.view(np.float32))
+    hb.rows(34, x_d[1:], rows, cols, cols, EPS, g_d[3:], y=y_d[2:], ctx=gpu)
+    got = y_d[2:].cpu().numpy().view(np.uint32).reshape(rows, cols)
+    check(got, oracle_rows(34, x, cols, EPS, gamma=gamma))
 
 
 def test_rmsnorm_feeds_a_linear_layer(gpu):
