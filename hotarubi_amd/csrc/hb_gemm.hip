@@ -704,6 +704,19 @@ namespace {
 // parallelism gains); 32 workgroups, or no split, lost 50-70% at M = 141.
 constexpr uint32_t kSmallGrid = 128, kTargetWorkgroups = 128, kMinSplitSteps = 4;
 constexpr uint32_t kSplitMidRows = 1024, kSplitMidWork = 65536;
+
+// K splits of args' gx x gy tiles: as many as fit in one round of
+// kTargetWorkgroups workgroups.
+void PlanKSplits(GemmArgs& args) {
+  uint32_t nblocks = 0;
+  for (uint32_t p = 0; p < args.n_pieces; ++p) nblocks += args.piece_kb[p];
+  const uint32_t steps = (nblocks + 1) / 2, tiles = args.gx * args.gy;
+  const uint32_t want = kTargetWorkgroups > tiles ? kTargetWorkgroups / tiles : 1u;
+  uint32_t per = (steps + want - 1) / want;
+  per = per < kMinSplitSteps ? kMinSplitSteps : per;
+  args.splits = (steps + per - 1) / per;
+  args.split_steps = per;
+}
 }  // namespace
 
 hipError_t GrowWorkspace(Workspace& ws, size_t bytes, hipStream_t stream) {
@@ -847,37 +860,41 @@ hipError_t LaunchLinear(const GemmArgs& in, uint32_t batch, bool fast, Workspace
   // even, 1024 x 2560 x 960 34.3 against 28.9 us).
   uint32_t blocks = 0;
   for (uint32_t p = 0; p < args.n_pieces; ++p) blocks += args.piece_kb[p];
-  if (small && args.quads * 4 <= kSplitMidRows &&
-      args.quads * 4 * blocks <= kSplitMidWork) {
-    SplitPlan(args);
-    args.fast_ep = 1u;
-    return LaunchSplitLinear(args, stream);
-  }
   args.fast_ep = 1u;
-  // Over panels the streaming kernel takes plain batched layers (and
-  // MXFP8); a plain single layer takes the panel kernel, whose 8 waves per
-  // CU hide more latency where a workgroup has one or two tiles (measured,
-  // one layer per launch: 1,600 x 2,048 x 736 24.0 -> 16.9 us, 4,512 x
-  // 2,560 x 960 48.7 -> 36.2 us, 14,848 x 256 x 1,024 26.6 -> 18.6 us,
-  // 67,584 x 64 x 576 47.5 -> 40.9 us).  Layers with ops or the requantize
-  // stay on the tile kernel: its epilogue runs on 16 waves per CU, the
-  // streaming kernel's on 4 (measured on the SparseDrive backbone's layers,
-  // e.g. 67,584 x 256 x 128 with bias, ReLU and the requantize: 55 against
-  // 139 us).
+  // (MXFP4 layers the wave kernel can take keep these tiles up to two a CU:
+  // 513 x 960, K 800, 510 tiles, 8.8 against 9.7 us; 300 x 2,560, K 960, 800
+  // tiles, 16.4 against 10.4 us)
+  const uint32_t wave_columns = WaveColumns(args, batch);
+  const bool mid = small && args.quads * 4 <= kSplitMidRows &&
+                   args.quads * 4 * blocks <= kSplitMidWork;
+  if (mid) {
+    GemmArgs split = args;
+    SplitPlan(split);
+    if (wave_columns == 0 || (uint64_t)split.gx * split.gy <= 2ull * DeviceCus())
+      return LaunchSplitLinear(split, stream);
+  }
+  if (wave_columns != 0) {
+    // The wave kernel needs no scratch; a fixed buffer keeps the limit it has
+    // always put on layers of this size (the K splits' partial sums).
+    if (fixed != nullptr && small && !mid) {
+      GemmArgs split = args;
+      PlanKSplits(split);
+      if (split.splits > 1) {
+        fixed->need = kSplitCounterBytes + WorkspaceBytes(split);
+        if (fixed->need > fixed->bytes || fixed->ptr == nullptr) return hipErrorOutOfMemory;
+      }
+    }
+    return LaunchWave(args, batch, wave_columns, stream);
+  }
+  // What the wave kernel leaves: over panels the streaming kernel takes plain
+  // batched layers (and MXFP8), the panel kernel a plain single layer of a
+  // long fold (its 8 waves per CU hide more latency where a workgroup has one
+  // or two tiles).  Layers with ops or the requantize stay on the tile kernel:
+  // its epilogue runs on 16 waves per CU, the streaming kernel's on 4.
   if (!small && StreamEligible(args) && batch > 1)
     return LaunchStream(args, batch, stream);
   if (!small && PanelEligible(args)) return LaunchPanel(args, batch, stream);
-  if (small) {
-    // as many splits as fit in one round of kTargetWorkgroups workgroups
-    uint32_t nblocks = 0;
-    for (uint32_t p = 0; p < args.n_pieces; ++p) nblocks += args.piece_kb[p];
-    const uint32_t steps = (nblocks + 1) / 2;
-    const uint32_t want = kTargetWorkgroups > gx * gy ? kTargetWorkgroups / (gx * gy) : 1u;
-    uint32_t per = (steps + want - 1) / want;
-    per = per < kMinSplitSteps ? kMinSplitSteps : per;
-    args.splits = (steps + per - 1) / per;
-    args.split_steps = per;
-  }
+  if (small) PlanKSplits(args);
   if (args.splits <= 1) return LaunchLinearFast(args, batch, stream);
 
   // (the partial sums start after the split counters)

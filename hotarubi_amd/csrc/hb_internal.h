@@ -267,6 +267,11 @@ hipError_t LaunchLinearFast(const GemmArgs& args, uint32_t batch, hipStream_t st
 // (no ops, no requantize, no K splits); `args` carries the tile grid.
 bool Fp4Eligible(const GemmArgs& args, uint32_t tile_rows);
 hipError_t LaunchFp4(const GemmArgs& args, hipStream_t stream);
+// MXFP4 layers of independent waves (hb_wave.hip): one piece, every
+// epilogue.  WaveColumns: the columns of a wave's tile (128 or 64), or 0 where
+// another kernel takes the launch.
+uint32_t WaveColumns(const GemmArgs& args, uint32_t batch);
+hipError_t LaunchWave(const GemmArgs& args, uint32_t batch, uint32_t columns, hipStream_t stream);
 // Streaming kernel over weight panels (hb_panel.hip): fast MXFP4, plain
 // layers of more than 64 rows, one piece over every block.
 bool PanelEligible(const GemmArgs& args);
