@@ -23,7 +23,10 @@ struct hb_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   bool own_stream = false;
-  uint32_t* d_flag = nullptr;  // device flag word for hb_encode_mxint8
+  uint32_t* d_flag = nullptr;  // device flag word of the preparation kernels
+  // hb_encode_*'s flag: pinned host memory that the kernel writes only for
+  // bad input, so a call clears and reads it without a memset or a copy
+  uint32_t* h_flag = nullptr;
   hb::Workspace ws;            // split partials / deferred epilogue inputs
 };
 
@@ -718,6 +721,9 @@ int hb_ctx_create(int device, hb_ctx** out) {
   ctx->device = device;
   hipError_t err = hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking);
   if (err == hipSuccess) err = hipMalloc(&ctx->d_flag, sizeof(uint32_t));
+  if (err == hipSuccess)
+    err = hipHostMalloc(reinterpret_cast<void**>(&ctx->h_flag), sizeof(uint32_t),
+                        hipHostMallocMapped | hipHostMallocPortable);
   // the workspace starts at the no-allocation path's size, so a layer whose
   // K splits fit in it never allocates after the context is created
   if (err == hipSuccess) err = hb::GrowWorkspace(ctx->ws, HB_NOALLOC_SCRATCH_BYTES, ctx->stream);
@@ -725,6 +731,7 @@ int hb_ctx_create(int device, hb_ctx** out) {
   if (err != hipSuccess) {
     hb::FreeWorkspace(ctx->ws);
     if (ctx->d_flag) (void)hipFree(ctx->d_flag);
+    if (ctx->h_flag) (void)hipHostFree(ctx->h_flag);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return HipFail(err, "context create");
@@ -739,6 +746,7 @@ int hb_ctx_destroy(hb_ctx* ctx) {
   (void)hipSetDevice(ctx->device);
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
   if (ctx->d_flag) (void)hipFree(ctx->d_flag);
+  if (ctx->h_flag) (void)hipHostFree(ctx->h_flag);
   hb::FreeWorkspace(ctx->ws);
   if (ctx->own_stream && ctx->stream) (void)hipStreamDestroy(ctx->stream);
   delete ctx;
@@ -1124,14 +1132,14 @@ namespace {
 int EncodeMx(hb_ctx* ctx, const float* x, uint32_t rows, uint32_t cols, void* out, bool fp8) {
   if (int rc = Enter(ctx)) return rc;
   if (!x || !out || rows < 1 || cols < 1) return Fail(HB_EINVAL, "bad encode arguments");
-  HB_HIP(hipMemsetAsync(ctx->d_flag, 0, sizeof(uint32_t), ctx->stream));
-  hipError_t err = hb::LaunchEncodeMxint8(x, rows, cols, static_cast<uint8_t*>(out),
-                                          ctx->d_flag, ctx->stream, fp8);
+  // (no launch that writes the flag is in flight: every call waits for its own)
+  volatile uint32_t* flag = ctx->h_flag;
+  *flag = 0;
+  const hipError_t err = hb::LaunchEncodeMxint8(x, rows, cols, static_cast<uint8_t*>(out),
+                                                ctx->h_flag, ctx->stream, fp8);
   if (err != hipSuccess) return HipFail(err, "encode launch");
-  uint32_t flag = 0;
-  HB_HIP(hipMemcpyAsync(&flag, ctx->d_flag, sizeof flag, hipMemcpyDeviceToHost, ctx->stream));
   HB_HIP(hipStreamSynchronize(ctx->stream));
-  if (flag) return Fail(HB_EINVAL, "%s input is infinite or NaN", fp8 ? "MXFP8" : "MXINT8");
+  if (*flag) return Fail(HB_EINVAL, "%s input is infinite or NaN", fp8 ? "MXFP8" : "MXINT8");
   return HB_OK;
 }
 
