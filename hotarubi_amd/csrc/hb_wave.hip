@@ -124,12 +124,15 @@ __global__ __launch_bounds__(64 * kWaves, 2) void WaveKernel(GemmArgs g) {
   uint32_t* c = g.c + z * g.c_batch;
   uint8_t* q_out = g.q_out ? g.q_out + z * g.q_batch : nullptr;
 
+  const uint32_t nblocks = g.piece_kb[0], first = g.piece_off[0], steps = (nblocks + 1) / 2;
   // The epilogue's small operands, which every wave shares: fetched first,
   // in LDS by the only barrier, which waits for them alone.
   constexpr int kActLoads = 512 / (64 * kWaves), kVecLoads = kMaxOps * 32 * kTN / (64 * kWaves);
-  // (no branch around a load: a value that no op reads comes from A's first
-  // bytes)
-  const uint64_t* act_src = g.tbuf != nullptr ? g.tbuf + 512 : reinterpret_cast<const uint64_t*>(a);
+  // (no branch around a load: a value that no op reads comes from the first
+  // A word of the fold; `a` itself may lie before the buffer, moved by the
+  // piece's place among the W blocks)
+  const uint8_t* const any = a + (size_t)first * kDdrWord;
+  const uint64_t* act_src = g.tbuf != nullptr ? g.tbuf + 512 : reinterpret_cast<const uint64_t*>(any);
   uint64_t act_v[kActLoads];
   uint32_t vec_v[kVecLoads];
   if (g.n_ops > 0) {  // uniform
@@ -142,12 +145,11 @@ __global__ __launch_bounds__(64 * kWaves, 2) void WaveKernel(GemmArgs g) {
       const uint32_t col = col0 + (threadIdx.x + 64 * kWaves * k) % (32 * kTN);
       const bool live = o < g.n_ops && (g.op_kind[o] == kEpAddP || g.op_kind[o] == kEpMulP);
       const uint32_t* src = live ? g.op_vec[o] + z * g.op_vec_batch[o]
-                                 : reinterpret_cast<const uint32_t*>(a);
+                                 : reinterpret_cast<const uint32_t*>(any);
       vec_v[k] = src[live && col < g.n ? col : 0u];
     }
   }
 
-  const uint32_t nblocks = g.piece_kb[0], first = g.piece_off[0], steps = (nblocks + 1) / 2;
   const uint32_t h = lane >> 5, l32 = lane & 31;
   const uint32_t quad = min((row0 + l32) >> 2, g.quads - 1);
   const uint32_t o_a = (quad * g.a_row + first) * kDdrWord, o_codes = (lane & 3) * 32;

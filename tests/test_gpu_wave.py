@@ -100,3 +100,35 @@ def test_wave_tiles(gpu, m, n, blocks, first, kb, layers, ops, panels):
             # the wave that saw the byte folds exactly; the fast ops are one
             # IEEE rounding each, as the engine's away from the range's ends
             assert np.array_equal(got[:32, :64], want[:32, :64])
+
+
+@pytest.mark.parametrize("panels", [False, True])
+@pytest.mark.parametrize("layers", [1, 3])
+def test_a_words_before_their_w_blocks(gpu, layers, panels):
+    """W blocks 16..19 of 20 against A words 0..3: the layer's A base, moved by
+    the piece's place, lies before A's first byte, and nothing may be read
+    there.  With vector ops and no table, whose unused loads take A's bytes."""
+    rng = np.random.default_rng(layers + 10 * panels)
+    m, n, kb, first, blocks = (1030 if layers == 1 else 170), 200, 20, 16, 4
+    a = [random_a_words(rng, m, blocks) for _ in range(layers)]
+    codes = [mxfp4_weights(rng, n, kb * 32) for _ in range(layers)]
+    w_d = dev(np.stack([oracle.pack_wbuf(*c) for c in codes]))
+    if panels:
+        packed = torch.empty((layers, hb.panel_bytes(n, kb)), dtype=torch.uint8, device=DEV)
+        for i in range(layers):
+            hb.pack_weights(w_d[i], n, kb, packed[i], ctx=gpu)
+        w_d = packed
+    bias = rng.standard_normal(n).astype(np.float32)
+    a_d, b_d = dev(np.stack(a)), dev(bias)
+    c = torch.zeros((layers, m, n), device=DEV)
+    descs = [hb.linear_desc(m, n, kb, a_d[i], [w_d[i]], [0], c[i], pieces=[(first, blocks, 0)],
+                            a_stride=blocks, ops=[(EP_ADDP, b_d), (EP_RELU, None)], mode=hb.FAST,
+                            panels=panels) for i in range(layers)]
+    print("A before its W blocks", (m, n, layers, panels), flush=True)
+    hb.linear_batched(descs, gpu)
+    torch.cuda.synchronize()
+    for i in range(layers):
+        w = oracle.pack_wbuf(*[x[..., first * (x.shape[-1] // kb):] for x in codes[i]])
+        want, _ = oracle_linear_mt(m, n, blocks, a[i], [w], [0],
+                                   ops=[(EP_ADDP, bias.view(np.uint32)), (EP_RELU, None)])
+        check_fast(c[i].cpu().numpy().view(np.uint32), want)
