@@ -873,19 +873,7 @@ hipError_t LaunchLinear(const GemmArgs& in, uint32_t batch, bool fast, Workspace
     if (wave_columns == 0 || (uint64_t)split.gx * split.gy <= 2ull * DeviceCus())
       return LaunchSplitLinear(split, stream);
   }
-  if (wave_columns != 0) {
-    // The wave kernel needs no scratch; a fixed buffer keeps the limit it has
-    // always put on layers of this size (the K splits' partial sums).
-    if (fixed != nullptr && small && !mid) {
-      GemmArgs split = args;
-      PlanKSplits(split);
-      if (split.splits > 1) {
-        fixed->need = kSplitCounterBytes + WorkspaceBytes(split);
-        if (fixed->need > fixed->bytes || fixed->ptr == nullptr) return hipErrorOutOfMemory;
-      }
-    }
-    return LaunchWave(args, batch, wave_columns, stream);
-  }
+  if (wave_columns != 0) return LaunchWave(args, batch, wave_columns, stream);
   // What the wave kernel leaves: over panels the streaming kernel takes plain
   // batched layers (and MXFP8), the panel kernel a plain single layer of a
   // long fold (its 8 waves per CU hide more latency where a workgroup has one

@@ -289,10 +289,12 @@ typedef struct hb_linear_desc {
   uint32_t a_stride;
 } hb_linear_desc;
 
-/* A single small layer (fewer than 128 output tiles) splits its K range
- * over workgroups in the context's workspace, which hb_ctx_create sizes to
+/* A single fast layer of more than 1,024 rows on few output tiles may split
+ * its K range over workgroups (hb_linear_noalloc_async names which) in the
+ * context's workspace, which hb_ctx_create sizes to
  * HB_NOALLOC_SCRATCH_BYTES; a layer that needs more grows it on its first
- * call of that shape (a hipMalloc, with no stream synchronization).  A workspace buffer is never freed before
+ * call of that shape (a hipMalloc, with no stream synchronization).  A
+ * workspace buffer is never freed before
  * hb_ctx_destroy, so work already queued and HIP graphs captured earlier
  * stay valid when a later call grows it; a graph is valid until its context
  * is destroyed.  Warm a shape up before capturing it in a graph (the
@@ -323,15 +325,15 @@ int hb_linear_group_async(hb_ctx* ctx, const hb_linear_desc* descs, uint32_t cou
 /* hb_linear_batched_async without any device allocation.  No counterpart in
  * the reference: it is for callers that cannot allocate device memory (code
  * under HIP graph capture, serving loops and harnesses that forbid
- * hipMalloc).  The partial sums and slow flags of a small layer's K splits
- * across workgroups (fast layers of more than 1,024 rows on few tiles),
- * which hb_linear keeps in the
- * context's growable workspace, go to a fixed per-device scratch array of
- * HB_NOALLOC_SCRATCH_BYTES instead
- * (resolved when a context is created on the device, held until the
- * process ends).  A layer that needs more returns HB_ENOMEM, naming the
- * size; every other argument rule is hb_linear_batched_async's.  All calls
- * on one GPU share that GPU's array and leave their partials in it:
+ * hipMalloc).  The partial sums and slow flags of K splits across workgroups
+ * (fast layers of more than 1,024 rows on few tiles: W8 over DDR words or
+ * weight panels, several pieces, or a long MXFP4 fold), which hb_linear keeps in
+ * the context's growable workspace, go to a fixed per-device scratch array
+ * of HB_NOALLOC_SCRATCH_BYTES instead (resolved when a context is created
+ * on the device, held until the process ends).  A layer whose K splits need
+ * more returns HB_ENOMEM, naming the size; every other layer needs none.
+ * Every other argument rule is hb_linear_batched_async's.  All calls on one
+ * GPU share that GPU's array and leave their partials in it:
  * calls that overlap in time on one GPU (different streams or contexts)
  * race, so serialize them. */
 
