@@ -179,6 +179,64 @@ def test_widths_and_special_rows(gpu, entry, cols, special):
                                quantize=quantize))
 
 
+# Every finite source and -infinity stays on softmax's plain passes: masks of
+# the type's lowest value, of -1e30 and of -infinity, rows whose largest is a
+# mask or near the type's highest, differences that overflow, subnormals and
+# sources near 2^-126; NaN, +infinity and an all -infinity row among them take
+# the guarded passes.  8,197 x 192 is the 16-lane, 3-unit layout.
+@pytest.mark.parametrize("rows,cols,valid", [(61, 64, 64), (61, 192, 187), (61, 776, 776),
+                                             (8197, 192, 192), (8197, 160, 155)])
+def test_softmax_masks(gpu, rows, cols, valid):
+    rng = np.random.default_rng(300 + rows + cols)
+    x = activations(rng, rows, cols, 4.0).view(np.float32)
+    lowest = np.finfo(np.float32).min
+    for r in range(rows):
+        kind = r % 16
+        pick = rng.random(cols) < 0.5
+        if kind < 4:
+            x[r, pick] = (lowest, np.float32(-1e30), -np.inf, np.float32(-1e4))[kind]
+        elif kind == 4:
+            x[r] = lowest
+        elif kind == 5:
+            x[r, pick], x[r, 0] = lowest, -lowest
+        elif kind == 6:
+            x[r] *= np.float32(1e-38)
+        elif kind == 7:
+            x[r] *= np.float32(2.0 ** -125)
+        elif kind == 8:
+            x[r] *= np.float32(1e37)
+        elif kind == 9 and r % 32 == 9:
+            x[r, 1] = (np.nan, np.inf, -np.nan)[r // 32 % 3]
+        elif kind == 10 and r % 32 == 10:
+            x[r] = -np.inf
+        elif kind == 11:
+            x[r] = np.where(pick, 0.0, -0.0)
+    x[:, valid:] = np.float32(np.nan)
+    tb = helpers.activation_table("silu")
+    for quantize in ((False, True) if cols % 32 == 0 else (False,)):
+        got = run_rows(gpu, 12, x.view(np.uint32), valid, tbuf=tb, quantize=quantize)
+        check(got, oracle_rows(12, x.view(np.uint32), valid, 0, tbuf=tb, quantize=quantize))
+
+
+# The 16-lane, 3-unit layout (132 to 192 columns past 8,192 rows) for the
+# norms: its 3-word accumulators, and the guarded passes from it.
+@pytest.mark.parametrize("entry,cols", [(34, 136), (34, 192), (22, 160), (22, 192)])
+def test_norms_past_8192_rows(gpu, entry, cols):
+    rng = np.random.default_rng(entry + cols)
+    rows = 8197
+    x = activations(rng, rows, cols, 4.0)
+    odd = np.flatnonzero(rng.random(rows) < 0.02)
+    x[odd[0::4], 3] = 0x7FC00000
+    x[odd[1::4], 7] = 0xFF800000
+    x[odd[2::4]] = (np.float32(1e-20) * x[odd[2::4]].view(np.float32)).view(np.uint32)
+    x[odd[3::4], ::2] = 0x00000010  # subnormals
+    gamma = helpers.random_fp32_words(rng, (cols,), 120, 130)
+    beta = helpers.random_fp32_words(rng, (cols,), 110, 130) if entry == 22 else None
+    for quantize in ((False, True) if cols % 32 == 0 else (False,)):
+        got = run_rows(gpu, entry, x, cols, EPS, gamma=gamma, beta=beta, quantize=quantize)
+        check(got, oracle_rows(entry, x, cols, EPS, gamma=gamma, beta=beta, quantize=quantize))
+
+
 def test_rows_off_16_byte_boundaries(gpu):
     rng = np.random.default_rng(3)
     rows, cols = 30, 96
