@@ -861,18 +861,22 @@ hipError_t LaunchLinear(const GemmArgs& in, uint32_t batch, bool fast, Workspace
   uint32_t blocks = 0;
   for (uint32_t p = 0; p < args.n_pieces; ++p) blocks += args.piece_kb[p];
   args.fast_ep = 1u;
-  // (MXFP4 layers the wave kernel can take keep these tiles up to two a CU:
+  // MXFP4 layers the wave kernel can take keep these tiles up to two a CU:
   // 513 x 960, K 800, 510 tiles, 8.8 against 9.7 us; 300 x 2,560, K 960, 800
-  // tiles, 16.4 against 10.4 us)
-  const uint32_t wave_columns = WaveColumns(args, batch);
-  const bool mid = small && args.quads * 4 <= kSplitMidRows &&
-                   args.quads * 4 * blocks <= kSplitMidWork;
-  if (mid) {
-    GemmArgs split = args;
-    SplitPlan(split);
-    if (wave_columns == 0 || (uint64_t)split.gx * split.gy <= 2ull * DeviceCus())
-      return LaunchSplitLinear(split, stream);
+  // tiles, 15.2 against 9.2 us.  Up to three where they requantize (493 x
+  // 1,408, K 416, 704 tiles, 9.1 against 10.6 us; 863 x 1,024, K 64, 864
+  // tiles, 8.7 against 8.8 us) and for folds that the 8 splits shorten most
+  // (676 x 768, K 3072, 528 tiles, 21.0 against 23.1 us).
+  const uint32_t rows = args.quads * 4;
+  if (small && rows <= kSplitMidRows && rows * blocks <= kSplitMidWork) {
+    const uint32_t tiles = (args.n + 31) / 32 * ((rows + 31) / 32);
+    const uint32_t per_cu = args.q_out != nullptr || blocks > 70 ? 3 : 2;
+    if (tiles <= per_cu * (uint32_t)DeviceCus() || WaveColumns(args, batch) == 0) {
+      SplitPlan(args);
+      return LaunchSplitLinear(args, stream);
+    }
   }
+  const uint32_t wave_columns = WaveColumns(args, batch);
   if (wave_columns != 0) return LaunchWave(args, batch, wave_columns, stream);
   // What the wave kernel leaves: over panels the streaming kernel takes plain
   // batched layers (and MXFP8), the panel kernel a plain single layer of a

@@ -442,14 +442,40 @@ void Launch(const GemmArgs& args, hipStream_t stream) {
 // So: 64 columns a wave (3 waves to a SIMD, each converting A for half the
 // columns) while 128 columns would give fewer than one wave to two SIMDs or
 // the fold is under 4 steps.  Others: the split kernel's 32 x 32 tiles while
-// they are at most two to a CU (its K splits are parallel, a wave's fold is
-// not), K splits of large tiles for a long fold over few waves, and tiles
-// that share converted operands where a long fold over many waves is all
-// conversion, where 64 rows fill their tile, or where the weights of many
-// layers of up to 128 rows are the traffic (their one tile reads them once).
-// Plain batches over DDR words stay on their streaming kernel (hb_fast4.hip:
-// 200 layers of 128 x 2,048, K 736, 107.8 against 134.3 us; 40 of 200 x 256,
-// K 320, 10.1 against 9.5).
+// they are at most two or three to a CU (LaunchLinear; its K splits are
+// parallel, a wave's fold is not), K splits of large tiles for a long fold
+// over few waves, and tiles that share converted operands where a long fold
+// over many waves is all conversion, where 64 rows fill their tile, or where
+// the weights of many layers of up to 128 rows are the traffic (their one
+// tile reads them once).  Plain batches over DDR words stay on their
+// streaming kernel (hb_fast4.hip: 200 layers of 128 x 2,048, K 736, 107.8
+// against 134.3 us; 40 of 200 x 256, K 320, 10.1 against 9.5).
+//
+// The lines past that are for launches whose workgroups (4 waves) just miss
+// a round of the CUs, or whose columns just miss a tile; each with the times
+// on both sides (us: the other kernel / 128 / 64 columns):
+//   64 columns for at most 5 column tiles that 128 would leave a quarter
+//   empty: 9,894 x 160, K 992, requantized 18.9 / 20.4 / 15.1 (folds under 24
+//   steps: 12,241 x 160, K 2976 32.7 / 31.7 / 37.5)
+//   128 columns for a long fold that they fit in one round and 64 do not: 15
+//   layers of 144 x 768, K 3072 32.4 / 28.2 / 35.2
+//   the others for a long fold past one round, up to one and a half: 11
+//   layers of 391 x 736, K 2048 26.7 / 33.7 / 36.8
+//   the tile kernel where its 64-row tiles fill the one round that this
+//   kernel just misses: 1,589 x 2,560, K 960, requantized 22.0 / 26.4 / 25.9
+//   the tile kernel for requantized 64 columns and up to 4 steps over few
+//   waves: 1,141 x 64, K 128 8.2 / 9.5 / 8.7
+//   K splits from 24 steps on where the layer requantizes: 1,211 x 96, K
+//   1760 14.2 / 21.1 / 16.9
+//   the panel kernel (plain, whole 256-column tiles) where its rounds are
+//   nearly full or its one round is this kernel's second: 7,952 x 3,072, K
+//   768 40.9 / 43.6 / 58.9, 10,602 x 512, K 512 12.9 / 14.1 / 14.6 (but
+//   15,943 x 768, K 768, rounds 0.73 full, 27.2 / 24.3 / 29.6)
+// Over 6,031 calls of 8 us and more, drawn after these lines were set (17 to
+// 70,000 rows, K 32 to 3,072, 64 to 3,072 columns, up to 64 layers), 10 take
+// over 8% longer than on the other kernels (51 without the lines), the worst
+// 1.21 times as long (27 layers of 174 x 736, K 864, requantized 21.9 / 26.1
+// / 25.9), and the mean is 0.79 of theirs.
 uint32_t WaveColumns(const GemmArgs& args, uint32_t batch) {
   // one MXFP4 plane, one run of blocks (over panels from the start of a step:
   // a chunk's two blocks are one step's)
@@ -458,13 +484,32 @@ uint32_t WaveColumns(const GemmArgs& args, uint32_t batch) {
     return 0;
   const uint64_t cus = DeviceCus(), simds = 4 * cus;
   const uint64_t rows = args.quads * 4ull, cols = args.groups * 8ull;
+  const uint64_t cols128 = (cols + 127) / 128, cols64 = (cols + 63) / 64;
+  // waves, and workgroups, of 128 and 64 columns
   const uint64_t row_waves = (rows + kWaveRows - 1) / kWaveRows * batch;
-  const uint64_t wide = row_waves * ((cols + 127) / 128), narrow = row_waves * ((cols + 63) / 64);
+  const uint64_t wide = row_waves * cols128, narrow = row_waves * cols64;
+  const uint64_t row_groups = (rows + kWaves * kWaveRows - 1) / (kWaves * kWaveRows) * batch;
+  const uint64_t wide_groups = row_groups * cols128, narrow_groups = row_groups * cols64;
   const uint32_t steps = (args.piece_kb[0] + 1) / 2;
+  const bool quantize = args.q_out != nullptr, plain = args.n_ops == 0 && !quantize;
   if (rows <= 64 ? narrow > simds : steps >= 32 && wide >= simds) return 0;
   if (rows <= 128 && wide > 2 * simds) return 0;
-  if (batch > 1 && !args.w_panels && args.n_ops == 0 && args.q_out == nullptr) return 0;
-  if (batch == 1 && steps >= 32 && narrow < cus) return 0;
+  if (batch > 1 && !args.w_panels && plain) return 0;
+  if (batch == 1 && steps >= (quantize ? 24u : 32u) && narrow < cus) return 0;
+  if (quantize && cols <= 64 && steps <= 4 && narrow <= simds / 2) return 0;
+  if (steps >= 24 && wide_groups > cus && 2 * wide_groups <= 3 * cus) return 0;
+  const uint64_t tiles64 = (rows + 63) / 64 * ((cols + 255) / 256) * batch;
+  if (steps >= 12 && wide_groups > cus && 4 * wide_groups <= 5 * cus &&
+      16 * tiles64 >= 15 * cus && tiles64 <= cus)
+    return 0;
+  if (batch == 1 && steps >= 8 && steps <= 24 && cols % 256 == 0 && PanelEligible(args)) {
+    const uint64_t tiles = (rows + 127) / 128 * (cols / 256);
+    if (6 * tiles >= 5 * ((tiles + cus - 1) / cus * cus) ||
+        (tiles <= cus && wide_groups > cus && 10 * wide_groups <= 13 * cus))
+      return 0;
+  }
+  if (!plain && steps < 24 && 3 * cols64 <= 5 * cols128) return 64;
+  if (steps >= 24 && wide_groups <= cus && narrow_groups > cus) return 128;
   return cols <= 64 || wide < simds / 2 || steps < 4 ? 64 : 128;
 }
 

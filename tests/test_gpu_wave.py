@@ -32,12 +32,15 @@ def unaligned(x):
 
 
 # (m, n, blocks, first block, kb_total, layers): 64-column waves with partial
-# row and column tiles, one block, an odd count, a range of the blocks;
+# row and column tiles, one block, an odd count, a range of the blocks, at
+# most 5 column tiles over many rows (1,057 x 160: 3 of 64, not 2 of 128);
 # 128-column waves (at least 512 of them, 4 steps and more) with a partly used
-# last column tile.
-SHAPES = [(1030, 72, 1, 0, 1, 1), (1025, 64, 3, 0, 3, 1), (1057, 160, 6, 2, 9, 1),
+# last column tile, and for a fold of 24 steps that fits one round of the CUs
+# in 128 columns and not in 64 (15 layers of 132 x 640: 150 workgroups, not
+# 300).
+SHAPES = [(1030, 72, 1, 0, 1, 1), (1025, 64, 9, 0, 9, 1), (1057, 160, 6, 2, 9, 1),
           (2049, 96, 13, 0, 13, 1), (170, 200, 5, 0, 5, 3), (65, 416, 7, 0, 7, 43),
-          (97, 288, 8, 4, 13, 43)]
+          (97, 352, 8, 4, 13, 43), (132, 640, 48, 0, 48, 15)]
 
 
 @pytest.mark.parametrize("panels", [False, True])
