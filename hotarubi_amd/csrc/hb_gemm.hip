@@ -668,6 +668,8 @@ void LaunchTile(GemmArgs args, uint32_t batch, hipStream_t stream) {
 //   2048 x 768, W8 768    27 / 26 / 26     1 x 960, K 960      13 / 13 / 9
 //   4512 x 320, K 960     25 / 21 / 22     928 x 512, W8 512   21 / 22 / 11
 //   32 layers of 128 x 960, K 2560   60 / 51 / 85
+// Up to 32 rows, half of a larger tile would be padding: 54 layers of 16 x
+// 3,072, W8 768 91 / 92 / 78; 54 of 16 x 3,072, K 768 53 / 60 / 49.
 template <bool kLinear>
 hipError_t LaunchTiles(const GemmArgs& args, uint32_t batch, hipStream_t stream) {
   const uint64_t cus = DeviceCus(), cols = args.groups * 8ull, rows = args.quads * 4ull;
@@ -678,7 +680,8 @@ hipError_t LaunchTiles(const GemmArgs& args, uint32_t batch, hipStream_t stream)
   };
   const uint64_t t0 = time(32, 64, 130, 200), t1 = time(64, 96, 200, 400),
                  t2 = time(64, 128, 260, 460);
-  if (t0 <= t1 && t0 <= t2) LaunchTile<kLinear, Tile<32, 64, 2, 4, 4>>(args, batch, stream);
+  if (rows <= 32 || (t0 <= t1 && t0 <= t2))
+    LaunchTile<kLinear, Tile<32, 64, 2, 4, 4>>(args, batch, stream);
   else if (t1 <= t2) LaunchTile<kLinear, Tile<64, 96, 4, 2, 6>>(args, batch, stream);
   else LaunchTile<kLinear, Tile<64, 128, 2, 2, 4>>(args, batch, stream);
   return hipGetLastError();

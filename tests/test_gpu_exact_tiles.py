@@ -48,17 +48,52 @@ def run(ctx, m, n, kb, a, planes, modes, ops=(), pieces=None, onto=None, tbuf=No
     return c.cpu().numpy().view(np.uint32), q.cpu().numpy() if quantize else None
 
 
-# Tiles of 32 x 64 (4 blocks a stage; the small shapes), of 64 x 96 and of
-# 64 x 128 (2 blocks a stage; 3,100 x 448 and 2,060 x 736 choose them on 256
-# CUs), each with partial last rows and columns and block counts that leave
-# a partial last stage, an odd and an even number of stages.
-SHAPES = [(1, 8, 1), (33, 72, 4), (130, 264, 7), (5, 64, 13), (3100, 448, 3), (2060, 736, 5),
-          (4100, 328, 2)]
+def tile_of(m, n, layers=1):
+    """The tile LaunchTiles picks: the least of rounds of the CUs times a
+    tile's rate, or one tile's latency; 32 x 64 up to 32 rows."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    rows = (m + 3) // 4 * 4
+
+    def time(bm, bn, rate, latency):
+        return max(-(-(-(-rows // bm) * -(-n // bn) * layers) // cus) * rate, latency)
+    t = [time(32, 64, 130, 200), time(64, 96, 200, 400), time(64, 128, 260, 460)]
+    if rows <= 32 or t[0] <= min(t[1:]):
+        return (32, 64)
+    return (64, 96) if t[1] <= t[2] else (64, 128)
+
+
+def row_tiles(m, bm=64):
+    """The quads of the first, a middle and the last row tile."""
+    quads, per = (m + 3) // 4, bm // 4
+    tiles = -(-quads // per)
+    pick = sorted({0, tiles // 2, tiles - 1})
+    return np.concatenate([np.arange(t * per, min(quads, (t + 1) * per)) for t in pick])
+
+
+def check_rows(got, q, m, n, kb, a, planes, modes, quads, onto=None, **kw):
+    """Rows `quads` of the outputs, bitwise (a layer's rows are independent)."""
+    rows = (quads[:, None] * 4 + np.arange(4)).reshape(-1)
+    rows = rows[rows < m]
+    want, wq = oracle_linear_mt(len(rows), n, kb, a.reshape(-1, kb, 144)[quads].reshape(-1, 144),
+                                planes, modes, onto=None if onto is None else onto[rows],
+                                quantize=q is not None, **kw)
+    assert np.array_equal(got[rows], want)
+    if q is not None:
+        assert np.array_equal(q.reshape(-1, n // 32, 144)[quads], wq.reshape(-1, n // 32, 144))
+
+
+# Every tile, each with partial last rows and columns and block counts that
+# leave a partial last stage (of 4 blocks in the smallest, 2 in the others),
+# an odd and an even number of stages.
+SHAPES = [(1, 8, 1, (32, 64)), (33, 72, 4, (32, 64)), (130, 264, 7, (32, 64)),
+          (5, 64, 13, (32, 64)), (3100, 448, 3, (32, 64)), (2060, 736, 5, (64, 96)),
+          (4100, 328, 2, (64, 96)), (2306, 1256, 3, (64, 128)), (1597, 2552, 2, (64, 128))]
 
 
 @pytest.mark.parametrize("w8", [False, True])
-@pytest.mark.parametrize("m,n,kb", SHAPES)
-def test_tiles(gpu, m, n, kb, w8):
+@pytest.mark.parametrize("m,n,kb,tile", SHAPES)
+def test_tiles(gpu, m, n, kb, tile, w8):
+    assert tile_of(m, n) == tile
     rng = np.random.default_rng(m + n + kb)
     a = random_a_words(rng, m, kb)
     planes, modes = weights(rng, n, kb, w8)
@@ -73,9 +108,12 @@ def test_tiles(gpu, m, n, kb, w8):
 # one, in the last one only; everywhere; and beyond [70, 179], where the tile
 # folds in integers.
 @pytest.mark.parametrize("where", ["none", "first", "late", "last", "all", "unsafe"])
-@pytest.mark.parametrize("m,n,kb,w8", [(70, 104, 41, False), (3100, 448, 21, True),
-                                       (2060, 736, 22, False)])
-def test_activation_scales(gpu, m, n, kb, w8, where):
+@pytest.mark.parametrize("m,n,kb,w8,tile", [
+    (70, 104, 41, False, (32, 64)), (3100, 448, 21, True, (32, 64)),
+    (2060, 736, 22, False, (64, 96)), (2060, 736, 21, True, (64, 96)),
+    (2306, 1256, 22, False, (64, 128)), (2306, 1256, 19, True, (64, 128))])
+def test_activation_scales(gpu, m, n, kb, w8, tile, where):
+    assert tile_of(m, n) == tile
     rng = np.random.default_rng(len(where) * 100 + kb)
     a = random_a_words(rng, m, kb, 116, 135).reshape(-1, kb, 144)
     block = {"first": 0, "late": kb - 4, "last": kb - 1, "unsafe": kb - 1}.get(where)
@@ -91,20 +129,42 @@ def test_activation_scales(gpu, m, n, kb, w8, where):
     onto = random_fp32_words(rng, (m, n), 110, 135)
     print("scales", (m, n, kb, w8, where), flush=True)
     got, _ = run(gpu, m, n, kb, a, planes, modes, onto=onto)
-    want, _ = oracle_linear_mt(m, n, kb, a, planes, modes, onto=onto)
-    assert np.array_equal(got, want)
+    check_rows(got, None, m, n, kb, a, planes, modes, row_tiles(m), onto=onto)
 
 
 @pytest.mark.parametrize("w8", [False, True])
-def test_pieces(gpu, w8):
-    """Pieces of 1, 5, 2 and 8 blocks out of order: stages end with a piece."""
+@pytest.mark.parametrize("m,n,tile", [(90, 160, (32, 64)), (2060, 736, (64, 96)),
+                                      (2306, 1280, (64, 128))])
+def test_pieces(gpu, m, n, tile, w8):
+    """Pieces of 1, 5, 2 and 8 blocks out of order: stages end with a piece;
+    requantized (24, 16 and 32 units of 4 columns a row of the tile)."""
+    assert tile_of(m, n) == tile
     rng = np.random.default_rng(5)
-    m, n, kb, pieces = 90, 160, 16, [(3, 1), (8, 5), (0, 2), (6, 8)]
+    kb, pieces = 16, [(3, 1), (8, 5), (0, 2), (6, 8)]
     a = random_a_words(rng, m, kb, 100, 140)
     planes, modes = weights(rng, n, kb, w8)
     got, q = run(gpu, m, n, kb, a, planes, modes, pieces=pieces, quantize=True)
-    want, wq = oracle_linear_mt(m, n, kb, a, planes, modes, pieces=pieces, quantize=True)
-    assert np.array_equal(got, want) and np.array_equal(q, wq)
+    check_rows(got, q, m, n, kb, a, planes, modes, row_tiles(m), pieces=pieces)
+
+
+@pytest.mark.parametrize("w8", [False, True])
+@pytest.mark.parametrize("m", [5, 30])
+def test_many_layers_of_few_rows(gpu, m, w8):
+    """54 layers of 3,072 columns: 32-row tiles (larger ones would take fewer
+    rounds, half of them padding)."""
+    n, kb, layers = 3072, 3, 54
+    rng = np.random.default_rng(m + w8)
+    a = [random_a_words(rng, m, kb) for _ in range(layers)]
+    data = [weights(rng, n, kb, w8) for _ in range(2)]
+    a_d, c = dev(np.stack(a)), torch.zeros((layers, m, n), device=DEV)
+    planes = [dev(np.stack([data[i % 2][0][p] for i in range(layers)])) for p in range(1 + w8)]
+    hb.linear_batched([hb.linear_desc(m, n, kb, a_d[i], [p[i] for p in planes], data[0][1], c[i])
+                       for i in range(layers)], gpu)
+    torch.cuda.synchronize()
+    got = c.cpu().numpy().view(np.uint32)
+    for i in (0, 1, 27, 53):
+        want, _ = oracle_linear_mt(m, n, kb, a[i], data[i % 2][0], data[0][1])
+        assert np.array_equal(got[i], want), i
 
 
 # Every op with operands of every exponent (zeros of both signs, subnormals,
