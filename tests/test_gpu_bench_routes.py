@@ -3,21 +3,21 @@ them, against the oracle (tools/iss/gemm_array.cpp:112-149 folded as
 tools/compiler/kernels.cpp:343-395 emits a layer, epilogue per
 tools/iss/lane.cpp):
 
-  * batched MXFP4 M=128 K=2560 N=960 (the headline): one tile per workgroup
-    (2 layers) and the persistent multi-tile route (80 layers, 320 tiles);
+  * batched MXFP4 M=128 K=2560 N=960 (the headline): the split kernel's
+    tiles (2 layers) and the persistent multi-tile route (80 layers, 320
+    tiles);
   * batched M=1024 (10 layers, 320 tiles);
   * batched M=1 and M=16 (the skinny route with a layer index per workgroup),
     over DDR words and over weight panels (the bench's layout);
-  * the SparseDrive-S stage-1 im2col shape K=576 N=64 at 16,384 rows (128
-    row tiles: the streaming route, not the small-layer split), both modes;
+  * the SparseDrive-S stage-1 im2col shape K=576 N=64 at 16,384 rows (the
+    wave kernel), both modes;
   * the SigLIP-style W8 MLP, up 768->3072 with MULP, ADDP, GELU and the
     requantize and down 3072->768 with MULP and ADDP, at M=2048, both modes;
-  * SmolVLA prefix layers at batch 32 (M=4512: q with requantize and down
-    with the residual add on 96-row tiles, a two-piece layer on them, k with
-    requantize on 64-row tiles) and the action expert's layers
-    at batch 32 (M=1600: q with requantize, down with the residual add, both
-    K-split over 64-row tiles; the 720->2048 gate with ACT_MUL(up) and
-    requantize, 200 unsplit 64-row tiles);
+  * SmolVLA prefix layers at batch 32 (M=4512: q and k with requantize on the
+    wave kernel, down with the residual add and a two-piece layer on 96-row
+    tiles) and the action expert's layers at batch 32 (M=1600: q with
+    requantize, down with the residual add, the 720->2048 gate with
+    ACT_MUL(up) and requantize, all on the wave kernel);
   * A operands whose codes cover all 256 int8 values, -128 included, through
     every fast route and the exact kernel.
 
@@ -135,11 +135,13 @@ def test_skinny_batched(gpu, m, panels):
 
 @pytest.mark.parametrize("mode", [hb.FAST, hb.EXACT])
 def test_all_int8_codes_batched(gpu, mode):
-    """A covering all 256 codes: the streaming route (M=128, batched) and, in
-    exact mode, the exact tile kernel."""
-    batched_layers(gpu, 128, 256, 12, 3, range(3), mode, all_codes=True, seed=77)
+    """A covering all 256 codes: the streaming route (260 layers of 128 rows)
+    and, in exact mode, the exact tile kernel."""
+    layers, check = (260, (0, 130, 259)) if mode == hb.FAST else (3, range(3))
+    batched_layers(gpu, 128, 256, 12, layers, check, mode, all_codes=True, seed=77)
 
 
+# (48 rows: the split kernel's tiles)
 @pytest.mark.parametrize("m", [16, 48])
 def test_all_int8_codes_skinny(gpu, m):
     batched_layers(gpu, m, 256, 12, 2, range(2), hb.FAST, all_codes=True, seed=78 + m)
@@ -180,7 +182,7 @@ def single_layer(gpu, m, n, kb, w8, mode, ops_fn=None, quantize=False, tbuf=None
 
 
 @pytest.mark.parametrize("mode", [hb.FAST, hb.EXACT])
-def test_sparsedrive_stage1_shape_128_row_tiles(gpu, mode):
+def test_sparsedrive_stage1_shape(gpu, mode):
     single_layer(gpu, 16384, 64, 18, False, mode, seed=90, bound=True)
 
 
@@ -224,12 +226,12 @@ def test_prefix_b32_down_residual(gpu):
 
 
 def test_expert_b32_q_requantize(gpu):
-    """720 -> 960 at M=1600: 100 tiles of 64 rows, K split, epilogue kernel."""
+    """720 -> 960 at M=1600."""
     single_layer(gpu, 1600, 960, 23, False, hb.FAST, quantize=True, seed=98)
 
 
 def test_expert_b32_down_residual(gpu):
-    """2048 -> 720 at M=1600: 75 tiles of 64 rows, K split over 64 blocks."""
+    """2048 -> 720 at M=1600."""
     single_layer(gpu, 1600, 720, 64, False, hb.FAST,
                  lambda r, m, n: [(hb.EP_ADD, helpers.random_fp32_words(r, (m, n), 118, 128))],
                  seed=99)
@@ -242,11 +244,12 @@ def test_expert_b32_gate_act_mul_requantize(gpu):
 
 
 @pytest.mark.parametrize("m,n,kb,w8,quantize", [
-    (141, 960, 30, False, False),   # K-split path + epilogue kernel
-    (50, 2048, 23, False, False),   # skinny kernel, one layer of up to 64 rows
-    (4512, 960, 30, False, True),   # 128-row tile kernel, unsplit, requantize
-    (2048, 3072, 24, True, False),  # 128-row tile kernel, W8, unsplit
-    (200, 768, 24, True, False)])   # K-split path, W8
+    (141, 960, 30, False, False),   # single-launch split kernel
+    (50, 2048, 23, False, False),   # the same
+    (4512, 960, 30, False, True),   # wave kernel, requantize
+    (2048, 3072, 24, True, False),  # 128-row tile kernel, W8
+    (200, 768, 24, True, False),    # split kernel, W8
+    (1100, 512, 16, True, False)])  # K splits and the epilogue kernel, W8
 def test_all_int8_codes_single_layer(gpu, m, n, kb, w8, quantize):
     """A covering all 256 codes through the fast single-layer routes."""
     single_layer(gpu, m, n, kb, w8, hb.FAST, quantize=quantize, all_codes=True, seed=97 + m,

@@ -96,11 +96,13 @@ def test_batched_pieces_onto_ops_requantize(gpu, slow):
 
 
 def test_unaligned_output_of_a_streaming_layer(gpu):
-    """C 4 bytes past a 16-byte boundary: a batched MXFP4 layer of 128 rows
-    that would take the streaming kernel (16-byte stores) is still correct."""
+    """C 4 bytes past a 16-byte boundary: 260 layers of 128 rows (128-row
+    tiles, one to a CU) that would take the streaming kernel over DDR words
+    (16-byte stores) are still correct."""
     rng = np.random.default_rng(320)
-    layers, m, n, k = 2, 128, 256, 320
-    data = [make_layer(rng, m, n, k, False) for _ in range(layers)]
+    layers, m, n, k = 260, 128, 256, 96
+    sets = [make_layer(rng, m, n, k, False) for _ in range(3)]
+    data = [sets[i % 3] for i in range(layers)]
     kb, modes = data[0][0], data[0][3]
     a_all = dev(np.stack([d[1] for d in data]))
     w_all = dev(np.stack([d[2][0] for d in data]))
@@ -112,6 +114,7 @@ def test_unaligned_output_of_a_streaming_layer(gpu):
     say("unaligned C", dict(layers=layers, m=m, n=n))
     hb.linear_batched(descs, gpu)
     got = host(c_all).view(np.uint32)
-    for i, d in enumerate(data):
+    for i, d in enumerate(sets):
         want, _ = oracle_linear(m, n, kb, d[1], d[2], d[3])
         check_fast(got[i], want)
+        assert all(np.array_equal(got[j], got[i]) for j in range(i, layers, 3))

@@ -329,12 +329,14 @@ def test_batched_layers_with_epilogue(gpu, w8, mode, quantize):
 
 
 @pytest.mark.parametrize("w8", [False, True])
-def test_fast_batched_pieces_and_onto(gpu, w8):
-    """Fast mode over a piece list (the multi-piece kernel), starting from C,
+@pytest.mark.parametrize("m", [160, 198])
+def test_fast_batched_pieces_and_onto(gpu, m, w8):
+    """Fast mode over a piece list (the multi-piece kernels: the split
+    kernel's tiles up to 160 rows, the tile kernel above), starting from C,
     with rows and columns that leave partial tiles, batched.  Step 3 pairs
     block 19 with block 0 (a step's blocks out of memory order)."""
     rng = np.random.default_rng(63 + w8)
-    layers, m, n, k = 3, 160, 320, 640
+    layers, n, k = 3, 320, 640
     data = [make_layer(rng, m, n, k, w8) for _ in range(layers)]
     kb, modes = data[0][0], data[0][3]
     pieces = [(13, 7), (0, 5), (5, 8)]
@@ -356,10 +358,11 @@ def test_fast_batched_pieces_and_onto(gpu, w8):
         assert (np.abs(g - w) <= 1e-5 * row_scale).all(), float((np.abs(g - w) / row_scale).max())
 
 
-@pytest.mark.parametrize("m,k,pieces", [(130, 416, None), (257, 640, [(11, 3), (0, 6)])])
+@pytest.mark.parametrize("m,k,pieces", [(130, 416, None), (190, 416, None),
+                                        (257, 640, [(11, 3), (0, 6)])])
 def test_fast_batched_odd_blocks_partial_tiles(gpu, m, k, pieces):
-    """MXFP4 layers of more than 64 rows (128-row tiles) with an odd number
-    of K blocks (the last step's second block is padding), rows not a
+    """MXFP4 layers of more than 64 rows (the split kernel's tiles up to 160
+    rows, the tile kernel above) with an odd number of K blocks (the last step's second block is padding), rows not a
     multiple of 4 and a partly used last column tile, batched.  With the
     piece list, step 1 pairs block 13 with block 0."""
     rng = np.random.default_rng(66 + m)
@@ -437,13 +440,14 @@ def test_fast_out_of_window_scales_recompute_exactly(gpu, w8):
 
 @pytest.mark.parametrize("w8", [False, True])
 def test_fast_k_split_64_row_tiles_out_of_window(gpu, w8):
-    """1100 x 512 x 512: more than 1,024 rows on 36 tiles of 64 rows, so K
-    splits whose partial sums and window flags go to the epilogue kernel.
-    Rows 64..127 (the second row tile) carry an out-of-window scale byte:
-    that row tile recomputes exactly, bit for bit; the rest stays within
-    the fast-mode tolerance."""
+    """1100 x 512 x 512, W8, and 1100 x 264 x 2112, MXFP4 (33 steps over 175
+    waves of 32 x 64, fewer than CUs): more than 1,024 rows on 36 tiles of 64
+    rows, so K splits whose partial sums and window flags go to the epilogue
+    kernel.  Rows 64..127 (the second row tile) carry an out-of-window scale
+    byte: that row tile recomputes exactly, bit for bit; the rest stays
+    within the fast-mode tolerance."""
     rng = np.random.default_rng(66 + w8)
-    m, n, k = 1100, 512, 512
+    m, n, k = (1100, 512, 512) if w8 else (1100, 264, 2112)
     kb, a, planes, modes = make_layer(rng, m, n, k, w8)
     a = a.copy()
     a.reshape(-1, kb, 144)[16:32, 3, 128] = 60   # rows 64..127
@@ -455,18 +459,45 @@ def test_fast_k_split_64_row_tiles_out_of_window(gpu, w8):
     assert (np.abs(g - w) <= 1e-5 * row_scale).all()
 
 
+def test_fast_tile_kernel_whose_round_is_full(gpu):
+    """1589 x 2560 x 960 MXFP4, requantized: 250 tiles of 64 rows fill the one
+    round that 260 workgroups of waves would miss, so the tile kernel.  Rows
+    64..127 carry an out-of-window scale byte: that row tile is exact, bit for
+    bit.  The first, a middle and the last row tile are checked."""
+    rng = np.random.default_rng(68)
+    m, n, k = 1589, 2560, 960
+    kb, a, planes, modes = make_layer(rng, m, n, k, False)
+    a = a.copy()
+    a.reshape(-1, kb, 144)[16:32, 5, 128] = 60
+    bias = helpers.random_fp32_words(rng, (n,), 118, 124)
+    ops = [(hb.EP_ADDP, bias), (hb.EP_RELU, None)]
+    got, gq = run_linear(gpu, m, n, kb, a, planes, modes, ops, quantize=True, mode=hb.FAST)
+    gq = gq.reshape(-1, n // 32, 144)
+    for q0 in (0, 16, 192, 384):
+        q1 = min((m + 3) // 4, q0 + 16)
+        r0, r1 = 4 * q0, min(m, 4 * q1)
+        want, wq = helpers.oracle_linear_mt(r1 - r0, n, kb,
+                                            a.reshape(-1, kb, 144)[q0:q1].reshape(-1, 144),
+                                            planes, modes, ops, quantize=True)
+        if q0 == 16:
+            assert_bits(got[r0:r1], want)
+        helpers.check_fast(got[r0:r1], want, gq[q0:q1].reshape(-1, 144), wq)
+
+
 def test_fast_96_row_tiles_out_of_window(gpu):
-    """4512 x 960 x 960 MXFP4: 188 tiles of 96 rows (128-row tiles would
-    leave CUs idle, 64-row tiles take two rounds).  Rows 96..191 (the second
-    row tile) carry an out-of-window scale byte: that row tile recomputes
-    exactly, bit for bit; the rest stays within the fast-mode tolerance."""
+    """4512 x 960 x 960 MXFP4 in two pieces (one would take the wave kernel):
+    188 tiles of 96 rows (128-row tiles would leave CUs idle, 64-row tiles
+    take two rounds).  Rows 96..191 (the second row tile) carry an
+    out-of-window scale byte: that row tile recomputes exactly, bit for bit;
+    the rest stays within the fast-mode tolerance."""
     rng = np.random.default_rng(67)
     m, n, k = 4512, 960, 960
     kb, a, planes, modes = make_layer(rng, m, n, k, False)
     a = a.copy()
     a.reshape(-1, kb, 144)[24:48, 5, 128] = 60   # rows 96..191
-    got, _ = run_linear(gpu, m, n, kb, a, planes, modes, mode=hb.FAST)
-    want, _ = helpers.oracle_linear_mt(m, n, kb, a, planes, modes)
+    pieces = [(0, 13), (13, 17)]
+    got, _ = run_linear(gpu, m, n, kb, a, planes, modes, pieces=pieces, mode=hb.FAST)
+    want, _ = helpers.oracle_linear_mt(m, n, kb, a, planes, modes, pieces=pieces)
     assert_bits(got[96:192], want[96:192])
     g, w = got.view(np.float32).astype(np.float64), want.view(np.float32).astype(np.float64)
     row_scale = np.abs(w).max(axis=1, keepdims=True)

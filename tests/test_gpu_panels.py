@@ -4,12 +4,12 @@ words (tools/compiler/tensors.cpp:66-90) bit for bit, and linear layers over
 panels against the oracle's layer over the same weights as DDR words
 (tools/iss/gemm_array.cpp:112-149 folded as tools/compiler/kernels.cpp:
 343-395): exact mode bitwise, fast mode within the fast-mode tolerance, on
-every kernel route that reads panels (the panel streaming kernel batched and
-persistent, a partial last panel and odd block counts, from C, out-of-window
-scale bytes; the skinny kernel for batches of up to 16 rows; the single-launch
-split kernel for one layer of up to 160 rows, with ops, requantize and W8
-planes; the 128-row tile kernel and its K-split path; the exact tile
-kernel)."""
+every kernel route that reads panels (the streaming kernel for many layers
+or long folds, a partial last panel and odd block counts, from C,
+out-of-window scale bytes; the panel kernel for plain single layers; the
+skinny kernel for batches of up to 16 rows; the single-launch split kernel for
+one layer of up to 160 rows, with ops, requantize and W8 planes; the tile
+kernel; the exact tile kernel; the wave kernel has its own tests)."""
 from __future__ import annotations
 
 import numpy as np
@@ -53,8 +53,11 @@ def test_pack_rejects_bad_arguments(gpu):
         assert err.value.code == hb.HB_EINVAL
 
 
-# ---- the panel streaming kernel (fast, plain MXFP4, more than 64 rows) ----
+# ---- the streaming kernel (fast, plain MXFP4 batches of more than 64 rows):
+# layers of up to 128 rows in more than 2,048 waves of 32 rows x 128 columns,
+# and folds of 32 steps and more in at least 1,024 ----
 
+# (2 layers take the split kernel's tiles: 240 of them)
 @pytest.mark.parametrize("layers,check", [(2, (0, 1)), (80, (0, 1, 37, 79))])
 def test_headline_shape(gpu, layers, check):
     batched_layers(gpu, 128, 960, 80, layers, check, hb.FAST, seed=layers + 500, panels=True)
@@ -64,26 +67,61 @@ def test_m1024_batched(gpu):
     batched_layers(gpu, 1024, 960, 80, 10, (0, 9), hb.FAST, seed=501, panels=True)
 
 
-@pytest.mark.parametrize("m,n,kb", [(128, 72, 3), (200, 320, 23), (131, 200, 5)])
-def test_partial_panels_odd_blocks(gpu, m, n, kb):
+@pytest.mark.parametrize("m,n,kb,layers", [(128, 72, 3, 520), (200, 320, 65, 50),
+                                           (131, 200, 67, 104)])
+def test_partial_panels_odd_blocks(gpu, m, n, kb, layers):
     """n not a multiple of 64 (a partial last panel; with n = 72 three of a
     tile's four waves have no columns), odd block counts (the last step's
     second block is padding), rows past a 128-row tile, many tiles."""
-    batched_layers(gpu, m, n, kb, 40, (0, 17, 39), hb.FAST, seed=m + n + kb, panels=True)
+    batched_layers(gpu, m, n, kb, layers, (0, 17, layers - 1), hb.FAST, seed=m + n + kb,
+                   panels=True)
 
 
 def test_onto_and_all_codes(gpu):
-    batched_layers(gpu, 128, 256, 12, 3, range(3), hb.FAST, all_codes=True, seed=502,
+    batched_layers(gpu, 128, 256, 12, 260, (0, 1, 130, 259), hb.FAST, all_codes=True, seed=502,
                    panels=True, onto=True)
 
 
 def test_out_of_window_scales_take_the_exact_fold(gpu):
-    batched_layers(gpu, 128, 320, 10, 4, range(4), hb.FAST, seed=503, panels=True,
+    batched_layers(gpu, 128, 320, 10, 172, (0, 1, 90, 171), hb.FAST, seed=503, panels=True,
                    bad_scales=True)
 
 
-def test_single_layer_many_tiles(gpu):
+def test_single_layer_many_rows(gpu):
     single_layer(gpu, 16384, 64, 18, False, hb.FAST, seed=504, bound=True, panels=True)
+
+
+# ---- the panel kernel: plain single layers whose 128 x 256 tiles fit rounds
+# of the 256 CUs better than waves of 32 x 128 do (n a multiple of 256, 8 to
+# 24 steps: one round where the waves take a second; rounds at least 5/6
+# full), and folds of 32 steps and more over at least 1,024 such waves ----
+
+# (m, n, blocks): 130 tiles, an odd block count; 428 tiles, two to a
+# workgroup; a partial last panel and tile, an odd number of steps
+@pytest.mark.parametrize("m,n,kb", [(16613, 256, 17), (13661, 1024, 16), (4101, 1000, 65)])
+@pytest.mark.parametrize("form", ["plain", "onto", "bad"])
+def test_panel_kernel(gpu, m, n, kb, form):
+    rng = np.random.default_rng(m + len(form))
+    a = helpers.random_a_words(rng, m, kb)
+    if form == "bad":  # rows 0..127: a scale byte outside the fast window
+        a.reshape(-1, kb, 144)[:32, kb - 1, 129] = 60
+    w = mxfp4_w(rng, n, kb)
+    onto = helpers.random_fp32_words(rng, (m, n), 118, 128) if form == "onto" else None
+    c_d = dev(onto.view(np.float32)) if form == "onto" else torch.zeros((m, n), device=DEV)
+    say("panel kernel", dict(m=m, n=n, kb=kb, form=form))
+    hb.linear(gpu, a=dev(a), planes=[to_panels(gpu, dev(w), n, kb)], modes=[0], c=c_d, m=m, n=n,
+              kb_total=kb, onto=form == "onto", mode=hb.FAST, panels=True)
+    got, quads = host(c_d).view(np.uint32), (m + 3) // 4
+    # the first, a middle and the last row tile (a layer's rows are independent)
+    for q0 in (0, quads // 64 * 32, (quads - 1) // 32 * 32):
+        r0, r1 = 4 * q0, min(m, 4 * q0 + 128)
+        part = a.reshape(-1, kb, 144)[q0:min(quads, q0 + 32)].reshape(-1, 144)
+        want, _ = helpers.oracle_linear_mt(r1 - r0, n, kb, part, [w], [0],
+                                           onto=None if onto is None else onto[r0:r1])
+        if form == "bad" and q0 == 0:
+            assert np.array_equal(got[:128], want)
+        else:
+            helpers.check_fast(got[r0:r1], want)
 
 
 # ---- the panel streaming kernel's persistent schedule: more tiles than CUs ----
@@ -206,8 +244,8 @@ def test_stream_many_tiles_exact_recompute_mid_stream(gpu):
 
 def test_stream_many_tiles_partial_panel(gpu):
     """N=200 (a partial last panel, three of a tile's five panels past the
-    layer) at M=1024 over 40 layers: 320 tiles."""
-    replicated_layers(gpu, 1024, 200, 5, 40, 3, range(3), seed=604)
+    layer) at M=1024 over 40 layers: 320 tiles, 33 steps."""
+    replicated_layers(gpu, 1024, 200, 65, 40, 3, range(3), seed=604)
 
 
 # ---- the other kernels over panels ----
@@ -225,7 +263,7 @@ def test_skinny_single(gpu, m, w8):
 @pytest.mark.parametrize("mode", [hb.FAST, hb.EXACT])
 def test_w8_ops_requantize(gpu, mode):
     """W8 planes as panels with MULP, ADDP, GELU and the requantize: the
-    128-row tile kernel (fast) and the exact tile kernel."""
+    single-launch split kernel (fast) and the exact tile kernel."""
     single_layer(gpu, 512, 3072, 24, True, mode, lambda r, m, n: per_channel(r, n, True),
                  quantize=True, tbuf=helpers.activation_table("gelu"), seed=509, panels=True)
 
@@ -233,9 +271,9 @@ def test_w8_ops_requantize(gpu, mode):
 @pytest.mark.parametrize("m", [141, 200])
 @pytest.mark.parametrize("mode", [hb.FAST, hb.EXACT])
 def test_small_layer_split_with_ops(gpu, mode, m):
-    """One small layer with the residual ADD: at 141 rows the single-launch
-    split kernel (fast), at 200 rows the 128-row tile kernel's K splits and
-    the epilogue kernel (fast); the deferred exact epilogue in exact mode."""
+    """One small layer with the residual ADD: the single-launch split kernel
+    (fast, up to 160 rows always, at 200 while its tiles are few) and the
+    exact tile kernel."""
     single_layer(gpu, m, 320, 30, False, mode,
                  lambda r, m, n: [(hb.EP_ADD, helpers.random_fp32_words(r, (m, n), 118, 128))],
                  seed=510 + m, panels=True)
@@ -267,7 +305,8 @@ def all_ops(rng, m, n):
             (hb.EP_RELU, None), (hb.EP_COPY, None)]
 
 
-def stream_ops(gpu, m, n, kb, ops_fn, seed, keep_c=True, onto=False, bad=False, fp8=False):
+def stream_ops(gpu, m, n, kb, ops_fn, seed, keep_c=True, onto=False, bad=False, fp8=False,
+               pieces=None):
     """One layer over panels with ops and the requantize, tiles enough to
     take the streaming kernel (at least one per CU); bad: a few weight
     scale bytes outside the fast window (their tiles are folded exactly,
@@ -288,10 +327,10 @@ def stream_ops(gpu, m, n, kb, ops_fn, seed, keep_c=True, onto=False, bad=False, 
                            bad=bad, fp8=fp8))
     hb.linear(gpu, a=dev(a), planes=[to_panels(gpu, dev(w), n, kb)], modes=[0], c=c_d, m=m, n=n,
               kb_total=kb, ops=dev_ops, tbuf=dev(tbuf.view(np.int64)), q_out=q_d, mode=hb.FAST,
-              panels=True, onto=onto, a_fp8=fp8)
+              panels=True, onto=onto, a_fp8=fp8, pieces=pieces)
     gq = host(q_d)
     want, wq = helpers.oracle_linear_mt(m, n, kb, a, [w], [0], ops=ops, tbuf=tbuf, quantize=True,
-                                        onto=c0, a_fp8=fp8)
+                                        onto=c0, a_fp8=fp8, pieces=pieces)
     if keep_c:
         helpers.check_fast(host(c_d).view(np.uint32), want)
     helpers.check_requantized(gq, wq)
@@ -323,9 +362,14 @@ def test_stream_ops_onto_mxfp8(gpu):
 
 @pytest.mark.parametrize("m", [4096, 4093])
 def test_tile_kernel_all_ops_requantize(gpu, m):
-    """MXINT8 layers with ops over panels take the 128-row tile kernel: every
-    op kind, C and the requantize."""
-    stream_ops(gpu, m, 2560, 5, all_ops, seed=630 + m)
+    """MXINT8 layers of several pieces with ops over panels take the 128-row
+    tile kernel: every op kind, C and the requantize."""
+    stream_ops(gpu, m, 2560, 5, all_ops, seed=630 + m, pieces=[(2, 3), (0, 2)])
+
+
+def test_wave_kernel_all_ops_requantize(gpu):
+    """The same layer in one piece: the wave kernel."""
+    stream_ops(gpu, 4093, 2560, 5, all_ops, seed=633)
 
 
 # ---- the skinny kernel over panels: batches of layers of up to 16 rows ----

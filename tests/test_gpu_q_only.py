@@ -21,7 +21,7 @@ pytestmark = pytest.mark.gpu
 
 
 def q_only(gpu, m, n, kb, mode, seed, w8=False, layers=1, ops=None, tbuf=None, panels=False,
-           w8_panels=False, fp8=False):
+           w8_panels=False, fp8=False, pieces=None):
     rng = np.random.default_rng(seed)
     a_h, w_h, w_d = [], [], []
     for _ in range(layers):
@@ -49,7 +49,8 @@ def q_only(gpu, m, n, kb, mode, seed, w8=False, layers=1, ops=None, tbuf=None, p
         q = torch.full((layers, qwords, 144), 0xA5, dtype=torch.uint8, device=DEV)
         descs = [hb.linear_desc(m, n, kb, a_d[i], w_d[i], modes, c[i] if with_c else None,
                                 ops=dev_ops, tbuf=tb_d, q_out=q[i], mode=mode, panels=panels,
-                                w8_panels=w8_panels, a_fp8=fp8) for i in range(layers)]
+                                w8_panels=w8_panels, a_fp8=fp8, pieces=pieces)
+                 for i in range(layers)]
         torch.cuda.synchronize()
         say("q only", dict(m=m, n=n, kb=kb, mode=mode, w8=w8, layers=layers, panels=panels,
                            w8_panels=w8_panels, fp8=fp8, with_c=with_c))
@@ -58,7 +59,7 @@ def q_only(gpu, m, n, kb, mode, seed, w8=False, layers=1, ops=None, tbuf=None, p
     assert np.array_equal(results[0], results[1])
     for i in (0, layers - 1):
         _, wq = helpers.oracle_linear_mt(m, n, kb, a_h[i], w_h[i], modes, ops=ops, tbuf=tbuf,
-                                         quantize=True, a_fp8=fp8)
+                                         quantize=True, a_fp8=fp8, pieces=pieces)
         if mode == hb.EXACT:
             assert np.array_equal(results[1][i], wq.reshape(qwords, 144))
         else:
@@ -70,23 +71,29 @@ def relu_bias(rng, n):
             (hb.EP_RELU, None)]
 
 
-def test_tile_kernel_128_rows(gpu):
-    """4512 x 960 x 960 MXFP4 (the SmolVLA prefix's q at B = 32): the
-    128-row tile kernel."""
+def test_wave_kernel_128_columns(gpu):
+    """4512 x 960 x 960 MXFP4 (the SmolVLA prefix's q at B = 32)."""
     q_only(gpu, 4512, 960, 30, hb.FAST, seed=900)
 
 
-def test_tile_kernel_panels_narrow_ops(gpu):
+def test_wave_kernel_panels_narrow_ops(gpu):
     """The backbone's stage-1 3x3 conv: 67,584 x 64 x 576 over panels, bias
     and ReLU."""
     q_only(gpu, 67584, 64, 18, hb.FAST, seed=901, panels=True,
            ops=relu_bias(np.random.default_rng(1), 64))
 
 
+@pytest.mark.parametrize("panels", [False, True])
+def test_tile_kernel_128_rows(gpu, panels):
+    """4096 x 2048 x 160 MXFP4 in two pieces: 256 tiles of 128 rows."""
+    q_only(gpu, 4096, 2048, 5, hb.FAST, seed=908, panels=panels, pieces=[(0, 2), (2, 3)],
+           ops=relu_bias(np.random.default_rng(5), 2048))
+
+
 def test_k_split_and_epilogue_kernel(gpu):
-    """1600 x 960 x 736: K split over workgroups, finished by the epilogue
-    kernel."""
-    q_only(gpu, 1600, 960, 23, hb.FAST, seed=902)
+    """1100 x 512 x 512, W8: 2 K splits over workgroups, finished by the
+    epilogue kernel."""
+    q_only(gpu, 1100, 512, 16, hb.FAST, seed=902, w8=True)
 
 
 def test_split_kernel(gpu):
@@ -101,8 +108,7 @@ def test_skinny_kernel_batched(gpu):
 
 @pytest.mark.parametrize("m", [200, 1000])
 def test_exact(gpu, m):
-    """Exact mode: the deferred epilogue of a small layer (200 rows) and the
-    exact tile kernel's own epilogue (1,000 rows), bias and ReLU."""
+    """Exact mode: the exact tile kernel's epilogue, bias and ReLU."""
     q_only(gpu, m, 320, 13, hb.EXACT, seed=905 + m, ops=relu_bias(np.random.default_rng(3), 320))
 
 
