@@ -4,9 +4,9 @@
 // in LDS.
 //
 // Arithmetic as in the other fast kernels: A as two exact FP6 E2M3 planes
-// h = fp6(q / 32) and (q - 32 h) / 2 with scale bytes ea - 1 and ea - 5, W's
-// E2M1 codes and E8M0 bytes untouched (hb_panel.hip); plane h, then plane r
-// of a step into each accumulator.
+// h = fp6(q / 32) and (q - 32 h) / 2 with scale bytes ea - 1 and ea - 5
+// (ring::SplitA), W's E2M1 codes and E8M0 bytes untouched (hb_panel.hip);
+// plane h, then plane r of a step into each accumulator.
 //
 // Why waves on their own.  Lane l of an A operand is row l % 32, block l / 32:
 // 32 consecutive bytes of a DDR word, so a lane loads and converts its own
@@ -19,10 +19,9 @@
 // again for every 128 columns (about 500 cycles a step against 256 of matrix
 // work), which is what bounds the wide layers; the narrow ones are bound by
 // HBM.
-#include <utility>
-
 #include "hb_device.h"
 #include "hb_internal.h"
+#include "hb_ring.h"
 
 namespace hb {
 namespace {
@@ -31,54 +30,11 @@ typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x6 __attribute__((ext_vector_type(6)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x32 __attribute__((ext_vector_type(32)));
 // 4 floats at any 4-byte address (operands and C of the caller's tensors)
 typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr uint32_t kSafeLo = 70, kSafeHi = 179;
 constexpr int kWaveRows = 32, kWaves = 4;
-
-template <typename Fn, int... kI>
-__device__ __forceinline__ void UnrollImpl(Fn&& f, std::integer_sequence<int, kI...>) {
-  (f(std::integral_constant<int, kI>{}), ...);
-}
-template <int kN, typename Fn>
-__device__ __forceinline__ void Unroll(Fn&& f) {
-  UnrollImpl(f, std::make_integer_sequence<int, kN>{});
-}
-
-// 32 int8 (8 dwords, K order) -> FP6 E2M3 codes of h = q/32 rounded and of
-// (q - 32h)/2, both exact (as in hb_panel.hip).  mask = 0 gives zeros.
-__device__ __forceinline__ void SplitA(const u32x4& x0, const u32x4& x1, uint32_t mask, i32x8& h8,
-                                       i32x8& r8) {
-  const f16x2 bias = {(_Float16)1152.0f, (_Float16)1152.0f};
-  f16x32 q;
-#pragma unroll
-  for (int d = 0; d < 8; ++d) {
-    const uint32_t u = ((d < 4 ? x0[d] : x1[d - 4]) & mask) ^ 0x80808080u;
-    const f16x2 p0 =
-        __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)) - bias;
-    const f16x2 p1 =
-        __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u)) - bias;
-    q[4 * d] = p0[0];
-    q[4 * d + 1] = p0[1];
-    q[4 * d + 2] = p1[0];
-    q[4 * d + 3] = p1[1];
-  }
-  const u32x6 h = __builtin_amdgcn_cvt_scalef32_pk32_fp6_f16(q, 32.0f);
-  const f16x32 hv = __builtin_amdgcn_cvt_scalef32_pk32_f16_fp6(h, 1.0f);
-  const f16x32 m32 = (_Float16)-32.0f;
-  const u32x6 r = __builtin_amdgcn_cvt_scalef32_pk32_fp6_f16(
-      __builtin_elementwise_fma(hv, m32, q), 2.0f);
-#pragma unroll
-  for (int i = 0; i < 6; ++i) {
-    h8[i] = (int)h[i];
-    r8[i] = (int)r[i];
-  }
-  h8[6] = h8[7] = r8[6] = r8[7] = 0;
-}
 
 // Largest value over the 8 lanes 8 p .. 8 p + 7 (xor 1, xor 2, half-row mirror).
 __device__ __forceinline__ uint32_t Max8(uint32_t x) {
@@ -215,7 +171,16 @@ __global__ __launch_bounds__(64 * kWaves, 2) void WaveKernel(GemmArgs g) {
 
   uint32_t bad = 0;
   auto convert = [&](const RawA& rw, PlanesA& p) __attribute__((always_inline)) {
-    SplitA(rw.a0, rw.a1, rw.mask, p.h, p.r);
+    const uint32_t x[8] = {rw.a0[0], rw.a0[1], rw.a0[2], rw.a0[3],
+                           rw.a1[0], rw.a1[1], rw.a1[2], rw.a1[3]};
+    ring::u32x6 h6, r6;
+    ring::SplitA(x, rw.mask, h6, r6);
+#pragma unroll
+    for (int i = 0; i < 6; ++i) {
+      p.h[i] = (int)h6[i];
+      p.r[i] = (int)r6[i];
+    }
+    p.h[6] = p.h[7] = p.r[6] = p.r[7] = 0;
     const uint32_t ea = __builtin_amdgcn_ubfe(rw.sa, 8 * (lane & 3), 8);  // row % 4 == lane % 4
     p.sa = (int)(((ea - 1u) & 0xFFu) | ((ea - 5u) << 8));
     bad |= (uint32_t)(ea - kSafeLo > kSafeHi - kSafeLo);
@@ -228,8 +193,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void WaveKernel(GemmArgs g) {
       const uint32_t ew = __builtin_amdgcn_ubfe((uint32_t)sw[t], kPanels ? 8 * (t % 2) : 0, 8);
       bad |= (uint32_t)(ew - kSafeLo > kSafeHi - kSafeLo);
     }
-    Unroll<2>([&](auto plane) {
-      Unroll<kTN>([&](auto jj) {
+    ring::Unroll<2>([&](auto plane) {
+      ring::Unroll<kTN>([&](auto jj) {
         constexpr int kJ = decltype(jj)::value, kP = decltype(plane)::value;
         const u32x4 wv = rw.w[kJ];
         const i32x8 b = {(int)wv[0], (int)wv[1], (int)wv[2], (int)wv[3], 0, 0, 0, 0};
@@ -368,7 +333,7 @@ __global__ __launch_bounds__(64 * kWaves, 2) void WaveKernel(GemmArgs g) {
         p = *reinterpret_cast<const f32x4_t*>(&lds_vec[o][32 * j + cc]);
       }
       // two rows' worth at a time: 16 table entries in flight would spill
-      Unroll<2>([&](auto hh) {
+      ring::Unroll<2>([&](auto hh) {
         constexpr int kB = decltype(hh)::value * 8;
         f32x8 v, x, pv;
 #pragma unroll
