@@ -344,19 +344,21 @@ __device__ __forceinline__ uint32_t SlowOutput(const GemmArgs& g, const uint8_t*
 // and 16x16 tile one MFMA with a zero accumulator gives s * 2^d exactly, and
 // the fold is an fma per output.
 //
-// Bound: the VALU beside the matrix cores.  A 16x16x32 MFMA takes 16.5
-// cycles and the 4 folds of its outputs as long; both together 23.3 where 3
-// waves of a SIMD take turns, 24.2 with 2, 37 with one (measured), so tiles
-// leave room for 2 or 3 workgroups per CU.  The rest is conversion: 5
-// instructions per 4 activations (an xor, two byte permutes, two packed f16
-// fmas; with bf16 operands, which have no packed arithmetic, it was 11) and
-// one per 2 FP4 weights.
+// Bound: no one unit.  A 16x16x32 MFMA takes 16.5 cycles and the 4 folds of
+// its outputs as long; both together 23.3 where 3 waves of a SIMD take turns,
+// 24.2 with 2, 37 with one (measured), so tiles leave room for 2 or 3
+// workgroups per CU, and a 64 x 96 tile costs a SIMD 140 cycles per block.
+// Next to that stands conversion: 5 instructions per 4 activations (an xor,
+// two byte permutes, two packed f16 fmas; with bf16 operands, which have no
+// packed arithmetic, it was 11) and one per 2 FP4 weights.  The K loop takes
+// about 1.6 times the cycles of both; the LDS moves 65 KB per 64 x 96 tile
+// and stage, 0.6 of its rate.
 //
 // Measured, one launch: 4512 x 960, K 2560, MXFP4 with the residual 129 -> 56
-// us; 2048 x 2304, K 768, W8 with MULP and ADDP 111 -> 45 us (bf16 operands,
-// 128 x 128 tiles of 4 waves, one block a barrier, and the ops in integers
-// before). The K loop now takes about 1.6 times its VALU and matrix-core
-// cycles; the LDS moves 65 KB per 64 x 96 tile and stage, 0.6 of its rate.
+// us (14 of them MFMAs and folds); 2048 x 2304, K 768, W8 with MULP and ADDP
+// 111 -> 45 us (8.5) (bf16 operands, 128 x 128 tiles of 4 waves, one block a
+// barrier, and the ops in integers before).  The 64 x 96 tile's 80 registers
+// spill 18 to 30 outside the MFMA loop (68 bytes a lane).
 //
 // The loop runs with the rows' factors fr left out, which are 1 for every
 // ea in [116, 135]; every kCheck stages it looks whether a row had another,

@@ -14,7 +14,6 @@ import torch
 
 import helpers
 import hotarubi_amd as hb
-import oracle
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -31,9 +30,7 @@ def dev(a):
 
 def layer(rng, m, n, kb):
     a = helpers.activations(rng, m, kb * 32)[1]
-    code, e = helpers.mxfp4_weights(rng, n, kb * 32)
-    w = oracle.pack_wbuf(code, e)
-    return a, w
+    return a, list(helpers.w8_planes_from_int8(rng.integers(-127, 128, (n, kb * 32))))
 
 
 def test_graph_survives_workspace_growth():
@@ -41,20 +38,22 @@ def test_graph_survives_workspace_growth():
     ctx = hb.Context(0)
     main = torch.cuda.current_stream()
     side = torch.cuda.Stream()
-    # small layer: 141 x 320 x 960 (4 tiles: K-split path, workspace ~1.5 MB)
-    m, n, kb = 141, 320, 30
+    # small layer: W8, 1,100 x 512 x 512 (36 tiles of 64 x 256, 2 K splits: 4.5
+    # MB of the 8 MiB the context starts with)
+    m, n, kb = 1100, 512, 16
     a, w = layer(rng, m, n, kb)
-    a_d, w_d = dev(a), dev(w)
+    a_d, w_d = dev(a), [dev(p) for p in w]
     c_d = torch.zeros((m, n), dtype=torch.float32, device=DEV)
-    desc = hb.linear_desc(m, n, kb, a_d, [w_d], [0], c_d, mode=hb.FAST)
-    want, _ = helpers.oracle_linear_mt(m, n, kb, a, [w], [0])
-    # larger small layer: 141 x 2048 x 2560 (16 tiles, workspace ~9 MB)
-    m2, n2, kb2 = 141, 2048, 80
+    desc = hb.linear_desc(m, n, kb, a_d, w_d, [1, 2], c_d, mode=hb.FAST)
+    want, _ = helpers.oracle_linear_mt(m, n, kb, a, w, [1, 2])
+    # larger small layer: 2,048 x 512 x 2,048 (64 tiles, 2 splits: 8 MiB of sums
+    # and the flags and counters, past the first buffer)
+    m2, n2, kb2 = 2048, 512, 64
     a2, w2 = layer(rng, m2, n2, kb2)
-    a2_d, w2_d = dev(a2), dev(w2)
+    a2_d, w2_d = dev(a2), [dev(p) for p in w2]
     c2_d = torch.zeros((m2, n2), dtype=torch.float32, device=DEV)
-    desc2 = hb.linear_desc(m2, n2, kb2, a2_d, [w2_d], [0], c2_d, mode=hb.FAST)
-    want2, _ = helpers.oracle_linear_mt(m2, n2, kb2, a2, [w2], [0])
+    desc2 = hb.linear_desc(m2, n2, kb2, a2_d, w2_d, [1, 2], c2_d, mode=hb.FAST)
+    want2, _ = helpers.oracle_linear_mt(m2, n2, kb2, a2, w2, [1, 2])
     try:
         say("warm up the small layer on the capture stream")
         with torch.cuda.stream(side):
